@@ -77,6 +77,18 @@ class NormDesc(ctypes.Structure):
     ]
 
 
+class GemmDesc(ctypes.Structure):
+    """Mirror of ``mvm_gemm_desc`` (include/mvm_gemm.h)."""
+
+    _fields_ = [
+        ("m", _i64), ("n", _i64), ("k", _i64), ("batch", _i64),
+        ("lda", _i64), ("ldb", _i64), ("ldc", _i64),
+        ("a_stride_batch", _i64), ("b_stride_batch", _i64), ("c_stride_batch", _i64),
+        ("b_seg", _i64), ("b_seg_stride", _i64),
+        ("a_kmajor", _i32), ("b_kmajor", _i32), ("accumulate", _i32), ("splits", _i32),
+    ]
+
+
 class AdamwTensor(ctypes.Structure):
     """Mirror of ``mvm_adamw_tensor`` (include/mvm_optim.h)."""
 
@@ -123,6 +135,13 @@ SIGNATURES = {
     "mvm_selftest_lanes": (ctypes.c_int, [_vp, _vp]),
 }
 
+# symbol -> (restype, argtypes) of include/mvm_gemm.h
+GEMM_SIGNATURES = {
+    "mvm_gemm_validate": (ctypes.c_int, [ctypes.POINTER(GemmDesc)]),
+    "mvm_gemm_workspace_bytes": (_i64, [ctypes.POINTER(GemmDesc)]),
+    "mvm_gemm_f32": (ctypes.c_int, [ctypes.POINTER(GemmDesc)] + [_vp] * 4 + [ctypes.c_size_t, _vp]),
+}
+
 _lib = None
 
 
@@ -143,7 +162,7 @@ def lib():
                 f"{LIB_PATH} is missing: build it with `python -m mlx_vision_mamba_amd.build` "
                 "(the HIP extension is required; there is no CPU fallback)")
         handle = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **GEMM_SIGNATURES}.items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args

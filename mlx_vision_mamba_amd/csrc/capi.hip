@@ -1,5 +1,5 @@
 // C ABI of libmvm_scan.so (declared in include/mvm_scan.h, mvm_conv.h,
-// mvm_norm.h and mvm_optim.h).
+// mvm_norm.h, mvm_gemm.h and mvm_optim.h).
 //
 // Host-side responsibilities: validate every argument before anything is
 // enqueued, pick the time-chunk length, carve the caller's workspace into
@@ -15,7 +15,9 @@
 #include <utility>
 
 #include "conv_kernels.h"
+#include "gemm_kernels.h"
 #include "mvm_conv.h"
+#include "mvm_gemm.h"
 #include "mvm_norm.h"
 #include "mvm_optim.h"
 #include "norm_kernels.h"
@@ -749,6 +751,104 @@ int mvm_layernorm_bwd(const mvm_norm_desc* desc, const float* x, const float* ga
                                          static_cast<float*>(workspace),
                                          static_cast<hipStream_t>(stream)),
                     "mvm_layernorm_bwd launch");
+}
+
+}  // extern "C"
+
+// ------------------------------------------------------------------- GEMM
+
+namespace {
+
+constexpr int64_t kGemmMaxDim = int64_t{1} << 30;
+constexpr int64_t kGemmMaxLd = int64_t{1} << 21;  // a tile's 32-bit offsets: up to 256 rows
+
+int check_gemm(const mvm_gemm_desc* d) {
+  if (d == nullptr) return fail(MVM_ERR_INVALID_ARG, "gemm desc is NULL");
+  if (d->m < 0 || d->n < 0 || d->k < 0 || d->batch < 0)
+    return fail(MVM_ERR_INVALID_ARG, "negative gemm size (m=%lld n=%lld k=%lld batch=%lld)",
+                (long long)d->m, (long long)d->n, (long long)d->k, (long long)d->batch);
+  if (d->m > kGemmMaxDim || d->n > kGemmMaxDim || d->k > kGemmMaxDim || d->batch > 65535)
+    return fail(MVM_ERR_UNSUPPORTED, "gemm size too large (m=%lld n=%lld k=%lld batch=%lld)",
+                (long long)d->m, (long long)d->n, (long long)d->k, (long long)d->batch);
+  if ((d->a_kmajor | d->b_kmajor | d->accumulate) & ~1)
+    return fail(MVM_ERR_INVALID_ARG, "gemm flags must be 0 or 1");
+  if (d->splits < 0 || d->splits > 64)
+    return fail(MVM_ERR_INVALID_ARG, "gemm splits=%d must be 0..64", d->splits);
+  const int64_t st[] = {d->lda, d->ldb, d->ldc, d->a_stride_batch, d->b_stride_batch,
+                        d->c_stride_batch, d->b_seg, d->b_seg_stride};
+  for (int64_t v : st)
+    if (v < 0) return fail(MVM_ERR_INVALID_ARG, "negative gemm stride");
+  if (d->b_seg > 0 && (d->b_seg % 32 != 0 || d->k % d->b_seg != 0))
+    return fail(MVM_ERR_INVALID_ARG, "gemm b_seg=%lld must be a multiple of 32 that divides k=%lld",
+                (long long)d->b_seg, (long long)d->k);
+  const int64_t bk = d->b_seg > 0 ? d->b_seg : d->k;
+  if (d->lda < (d->a_kmajor ? d->k : d->m) || d->ldb < (d->b_kmajor ? bk : d->n))
+    return fail(MVM_ERR_INVALID_ARG, "gemm leading dimension smaller than its row");
+  if (d->lda >= kGemmMaxLd || d->ldb >= kGemmMaxLd)
+    return fail(MVM_ERR_UNSUPPORTED, "gemm leading dimension exceeds %lld", (long long)kGemmMaxLd - 1);
+  if ((d->a_kmajor && (d->lda % 4 || d->a_stride_batch % 4)) ||
+      (d->b_kmajor && (d->ldb % 4 || d->b_stride_batch % 4 || d->b_seg_stride % 4)))
+    return fail(MVM_ERR_UNSUPPORTED, "a k-major gemm operand needs strides that are multiples of 4");
+  if (!no_overlap({{d->batch, d->c_stride_batch}, {d->m, d->ldc}, {d->n, 1}}))
+    return fail(MVM_ERR_INVALID_ARG, "gemm C strides overlap");
+  return MVM_OK;
+}
+
+// (after check_gemm) the launch geometry with its tile shape and split
+int gemm_geom(const mvm_gemm_desc* d, mvm::GemmGeom& g) {
+  g.M = static_cast<int32_t>(d->m); g.N = static_cast<int32_t>(d->n); g.K = static_cast<int32_t>(d->k);
+  g.batch = static_cast<int32_t>(d->batch);
+  g.lda = static_cast<int32_t>(d->lda); g.ldb = static_cast<int32_t>(d->ldb); g.ldc = d->ldc;
+  g.sa = d->a_stride_batch; g.sb = d->b_stride_batch; g.sc = d->c_stride_batch;
+  g.seg = static_cast<int32_t>(d->b_seg > 0 ? d->b_seg : std::max<int64_t>(d->k, 1));
+  g.seg_stride = d->b_seg > 0 ? d->b_seg_stride : 0;
+  g.a_km = d->a_kmajor; g.b_km = d->b_kmajor;
+  g.accumulate = d->accumulate;
+  g.nsplit = d->splits;
+  mvm::gemm_plan(g);
+  if (d->batch * g.nsplit > 65535 || ceil_div(d->m, 64) * ceil_div(d->n, 64) > INT32_MAX / 256)
+    return fail(MVM_ERR_UNSUPPORTED, "gemm grid too large (m=%lld n=%lld batch=%lld splits=%d)",
+                (long long)d->m, (long long)d->n, (long long)d->batch, g.nsplit);
+  return MVM_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int mvm_gemm_validate(const mvm_gemm_desc* desc) {
+  int rc = check_gemm(desc);
+  mvm::GemmGeom g;
+  if (rc == MVM_OK) rc = gemm_geom(desc, g);
+  return rc == MVM_OK ? ok() : rc;
+}
+
+int64_t mvm_gemm_workspace_bytes(const mvm_gemm_desc* desc) {
+  int rc = check_gemm(desc);
+  mvm::GemmGeom g;
+  if (rc == MVM_OK) rc = gemm_geom(desc, g);
+  if (rc != MVM_OK) return rc;
+  return static_cast<int64_t>(align_up(sizeof(float) * mvm::gemm_partial_floats(g)));
+}
+
+int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, float* C,
+                 void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_gemm(desc);
+  mvm::GemmGeom g;
+  if (rc == MVM_OK) rc = gemm_geom(desc, g);
+  if (rc != MVM_OK) return rc;
+  if (g.M == 0 || g.N == 0 || g.batch == 0 || (g.K == 0 && g.accumulate)) return ok();
+  if (!C || (g.K > 0 && (!A || !B))) return fail(MVM_ERR_INVALID_ARG, "mvm_gemm_f32: NULL pointer");
+  if ((g.a_km && (reinterpret_cast<uintptr_t>(A) & 15u)) || (g.b_km && (reinterpret_cast<uintptr_t>(B) & 15u)))
+    return fail(MVM_ERR_INVALID_ARG, "mvm_gemm_f32: a k-major operand must be 16-byte aligned");
+  const size_t need = align_up(sizeof(float) * mvm::gemm_partial_floats(g));
+  if (need > 0) {
+    rc = check_ws("mvm_gemm_f32", workspace, workspace_bytes, need);
+    if (rc != MVM_OK) return rc;
+  }
+  return hip_status(mvm::launch_gemm(g, A, B, C, static_cast<float*>(workspace),
+                                     static_cast<hipStream_t>(stream)),
+                    "mvm_gemm_f32 launch");
 }
 
 }  // extern "C"

@@ -1,0 +1,477 @@
+// float32 matrix products for the block's projections on the bf16 matrix
+// units of gfx950 (in_proj / out_proj and their gradients,
+// mamba_block.py:125, :153, :165, :191).
+//
+// Why not the float32 matrix instructions: they reach 155 TFLOP/s on this
+// chip, the bf16 ones 1,700-1,800 from registers.  Every float32 x is the
+// exact sum of three bf16 values
+//   hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid    (round to nearest)
+// (24 = 8 + 8 + 8 significand bits), and
+//   a b = hi hi + (hi mid + mid hi) + (mid mid + hi lo + lo hi) + r,
+// |r| <= 2^-25 |a b| at the most and about 2^-28 on average: six bf16 products stand for
+// one float32 product, ~290 TFLOP/s at best.  The products of bf16 values
+// are exact in float32, and a 32x32x16 MFMA rounds the sum of its 16 less
+// often than 16 float32 FMAs do.
+//
+// hi hi has an accumulator of its own.  The matrix unit cuts off, downwards,
+// what lies far below the accumulator: with the small products added to the
+// same one, C came out low by 2e-8 of its rms (k = 384) whatever its sign,
+// invisible in C's own error but not in later sums over its rows (a block's
+// x_proj weight gradient: 4e-5 instead of 3e-6).  Apart, the mean error is
+// that of the float32 instructions (3e-10), and the error in the 2-norm
+// against float64 1.1e-7 at k = 384 and 2.7e-7 at k = 6144 in 3 parts (normal
+// inputs; the BLAS library's float32 matrix instructions: 3.5e-7 and 1.4e-6).
+//
+// What the split cannot hold, and what is done: infinities and NaN (and
+// values above the largest bf16, which round to infinity) make a NaN out of
+// hi - hi, and below 2^-109 the low parts underflow.  A wave whose results
+// are not all finite, or all so small (below 2^-64, not all zero) that their
+// inputs may have been, computes its part of the tile again with the float32
+// matrix instructions, which have neither limit.
+//
+// Work split: a 256-thread workgroup computes a BM x BN tile, its 4 waves
+// (2 x 2) a quarter each in 32x32x16 MFMA tiles.  Both operands are split
+// into their three bf16 planes once per workgroup, on the way from global
+// memory (held in registers two steps ahead) into double-buffered LDS; each
+// fragment read from LDS then feeds six MFMAs.  A thread holds 8 consecutive
+// k of one row, whichever way the operand lies in memory, so both layouts
+// arrive in LDS the same way.  The 16-byte chunks of a row are swapped by a
+// bit of the row so that neither the writes nor the fragment reads of 8
+// neighbouring lanes share a bank.
+// Bound: with the MFMAs alone the loop runs at 230-240 TFLOP/s; the
+// split's VALU work (11 instructions per pair of values), the LDS traffic and
+// the global loads take the rest: 143-161 TFLOP/s on in_proj and out_proj of
+// 6272-16384 rows, where the BLAS library's float32 kernels reach 95-137.
+// Scheduling barriers and raised wave priority around the MFMAs were both
+// slower (they keep the split's instructions from filling in between).
+//
+// Order of tiles: workgroups are dealt to the 8 XCDs in turn, so the tile
+// index is remapped to give each XCD one contiguous range, walked in groups
+// of 8 row tiles, whose operands stay in that XCD's L2.
+#include <algorithm>
+
+#include "gemm_kernels.h"
+#include "scan_common.h"
+
+namespace mvm {
+
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kGroupM = 8;  // row tiles per group of the tile order
+
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// the three bf16 planes of 8 values
+__device__ __forceinline__ void split8(const float (&v)[8], uint4 (&pl)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      w[q][i] = pack_bf16(a, b);
+      if (q < 2) {
+        a -= __uint_as_float(w[q][i] << 16);
+        b -= __uint_as_float(w[q][i] & 0xffff0000u);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) pl[q] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+}
+
+// One operand's share of a workgroup: ROWS rows (of A, or columns of B) by
+// BK values of k per step.  KM: k is the contiguous index.
+template <int ROWS, int BK, bool KM>
+struct Operand {
+  static constexpr int kChunks = BK / 8;
+  static constexpr int kItems = ROWS * kChunks / kThreads;  // 8-value items per thread
+  static_assert(kItems * kThreads == ROWS * kChunks, "items divide evenly");
+  int row[kItems], chunk[kItems];
+  uint32_t off[kItems];  // element offset of the item's first value from the step's base
+
+  // rows past `nrows` read the last row: their results are not stored
+  __device__ __forceinline__ void init(int tid, int nrows, int ld) {
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const int x = tid + kThreads * i;
+      row[i] = KM ? x / kChunks : x % ROWS;
+      chunk[i] = KM ? x % kChunks : x / ROWS;
+      const int r = row[i] < nrows ? row[i] : nrows - 1;
+      off[i] = KM ? r * ld + chunk[i] * 8 : chunk[i] * 8 * ld + r;
+    }
+  }
+  __device__ __forceinline__ void load(float (&v)[kItems][8], const float* __restrict__ base, int ld) const {
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      if constexpr (KM) {
+        const float4 x = *reinterpret_cast<const float4*>(base + off[i]);
+        const float4 y = *reinterpret_cast<const float4*>(base + off[i] + 4);
+        v[i][0] = x.x; v[i][1] = x.y; v[i][2] = x.z; v[i][3] = x.w;
+        v[i][4] = y.x; v[i][5] = y.y; v[i][6] = y.z; v[i][7] = y.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = (base + e * ld)[off[i]];
+      }
+    }
+  }
+  // the last, partial step: `left` < BK values of k remain; the others are
+  // read from the step's first value (in bounds) and replaced by zero
+  __device__ __forceinline__ void load_tail(float (&v)[kItems][8], const float* __restrict__ base, int ld,
+                                            int left) const {
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      const uint32_t r = off[i] - (KM ? chunk[i] * 8 : chunk[i] * 8 * ld);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int p = chunk[i] * 8 + e;
+        const float t = base[r + static_cast<uint32_t>(p < left ? (KM ? p : p * ld) : 0)];
+        v[i][e] = p < left ? t : 0.f;
+      }
+    }
+  }
+  // LDS position of a row's chunk: 8 neighbouring rows at one chunk cover
+  // all the 16-byte columns of 128 bytes
+  __device__ static __forceinline__ int swz(int r, int c) {
+    return BK == 16 ? (c ^ ((r >> 2) & 1)) * 8 : (c ^ ((r >> 1) & 3)) * 8;
+  }
+  __device__ __forceinline__ void store(uint16_t (*lds)[ROWS][BK], const float (&v)[kItems][8]) const {
+#pragma unroll
+    for (int i = 0; i < kItems; ++i) {
+      uint4 pl[3];
+      split8(v[i], pl);
+      const int o = swz(row[i], chunk[i]);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint4*>(&lds[q][row[i]][o]) = pl[q];
+    }
+  }
+};
+
+template <int BM, int BN, int BK, int OCC, bool AKM, bool BKM>
+__global__ void __launch_bounds__(kThreads, OCC)
+gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B,
+            float* __restrict__ C) {
+  constexpr int MT = BM / 64, NT = BN / 64;  // 32 x 32 tiles of a wave
+  __shared__ __attribute__((aligned(16))) uint16_t sA[2][3][BM][BK];
+  __shared__ __attribute__((aligned(16))) uint16_t sB[2][3][BN][BK];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ntm = (g.M + BM - 1) / BM, ntn = (g.N + BN - 1) / BN;
+  int tm, tn;
+  {
+    const int nt = ntm * ntn, bid = blockIdx.x;
+    const int per = nt / 8, rem = nt % 8, x = bid % 8;
+    const int t = x * per + min(x, rem) + bid / 8;  // XCD x owns one contiguous range
+    const int grp = t / (kGroupM * ntn), r = t % (kGroupM * ntn);
+    const int gm = min(kGroupM, ntm - grp * kGroupM);
+    tm = grp * kGroupM + r % gm;
+    tn = r / gm;
+  }
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int sp = blockIdx.z % g.nsplit, q = blockIdx.z / g.nsplit;
+  const int k0 = sp * g.kper, k1 = min(g.K, k0 + g.kper);
+  const int len = k1 - k0;  // may be <= 0 in the last parts: a zero product
+  const int full = len > 0 ? len / BK : 0;
+  // step bases, advanced by one step at a time; B moves to its next segment
+  // when it reaches the end of one
+  const float* Ab = A + q * g.sa + (AKM ? static_cast<int64_t>(m0) * g.lda + k0
+                                        : static_cast<int64_t>(k0) * g.lda + m0);
+  const int seg0 = k0 / g.seg;
+  int kin = k0 - seg0 * g.seg;
+  const float* Bb = B + q * g.sb + seg0 * g.seg_stride +
+                    (BKM ? static_cast<int64_t>(n0) * g.ldb + kin : static_cast<int64_t>(kin) * g.ldb + n0);
+  const float* const A0 = Ab;
+  const float* const B0 = Bb;
+  const int64_t astep = AKM ? BK : static_cast<int64_t>(BK) * g.lda;
+  const int64_t bstep = BKM ? BK : static_cast<int64_t>(BK) * g.ldb;
+  const int64_t bfix = g.seg_stride - (BKM ? g.seg : static_cast<int64_t>(g.seg) * g.ldb);
+  int pos = 0;
+  Operand<BM, BK, AKM> oa;
+  Operand<BN, BK, BKM> ob;
+  oa.init(tid, g.M - m0, g.lda);
+  ob.init(tid, g.N - n0, g.ldb);
+  float pa[2][oa.kItems][8], pb[2][ob.kItems][8];
+  // the next full step into register set r; past the last one it is read
+  // again (never used), so the main loop has no branches
+  auto prefetch = [&](int r) {
+    oa.load(pa[r], Ab, g.lda);
+    ob.load(pb[r], Bb, g.ldb);
+    if (pos + 1 < full) {
+      ++pos;
+      Ab += astep;
+      Bb += bstep;
+      kin += BK;
+      if (kin == g.seg) {
+        kin = 0;
+        Bb += bfix;
+      }
+    }
+  };
+  auto stage = [&](int buf, int r) {
+    oa.store(sA[buf], pa[r]);
+    ob.store(sB[buf], pb[r]);
+  };
+
+  // hi * hi, and the five smaller products (added at the end)
+  f32x16 acc[MT][NT] = {}, acs[MT][NT] = {};
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+  const int fr = lane & 31, fh = lane >> 5;
+  auto compute = [&](int buf) {
+#pragma unroll
+    for (int h = 0; h < BK / 16; ++h) {
+      const int fo = Operand<BM, BK, AKM>::swz(fr, 2 * h + fh);
+      bf16x8 b[3][NT];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          b[p][j] = *reinterpret_cast<const bf16x8*>(&sB[buf][p][wn + j * 32 + fr][fo]);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        bf16x8 a[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) a[p] = *reinterpret_cast<const bf16x8*>(&sA[buf][p][wm + i * 32 + fr][fo]);
+        constexpr int kPa[5] = {2, 0, 1, 1, 0}, kPb[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+        for (int t = 0; t < 5; ++t)
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            acs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kPa[t]], b[kPb[t]][j], acs[i][j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0][j], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  if (full > 0) {
+    prefetch(0);
+    prefetch(1);
+    stage(0, 0);
+    int s = 0;
+    for (; s + 1 < full; s += 2) {
+      __syncthreads();
+      prefetch(0);
+      compute(0);
+      stage(1, 1);
+      __syncthreads();
+      prefetch(1);
+      compute(1);
+      stage(0, 0);
+    }
+    if (s < full) {
+      __syncthreads();
+      compute(0);
+    }
+    __syncthreads();
+  }
+  if (len > full * BK) {  // (segments are whole steps: no segment ends in a partial one)
+    const int64_t done = full;
+    int64_t bo = done * bstep;
+    if (g.seg < g.K) bo += ((k0 + full * BK) / g.seg - seg0) * bfix;
+    oa.load_tail(pa[0], A0 + done * astep, g.lda, len - full * BK);
+    ob.load_tail(pb[0], B0 + bo, g.ldb, len - full * BK);
+    stage(0, 0);
+    __syncthreads();
+    compute(0);
+  }
+
+  // results the split cannot vouch for: again with the float32 instructions
+  float big = 0.f;
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        acc[i][j][r] += acs[i][j][r];
+        const float x = fabsf(acc[i][j][r]);
+        finite &= x < __builtin_inff();
+        big = fmaxf(big, x);
+      }
+  // (per wave, its quarter of the tile: no barrier below)
+  if (__ballot(!finite) != 0 || (__ballot(big > 0.f) != 0 && __ballot(big >= 0x1p-64f) == 0)) {
+    int ra[MT], rb[NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) ra[i] = min(wm + i * 32 + fr, g.M - 1 - m0);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) rb[j] = min(wn + j * 32 + fr, g.N - 1 - n0);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = f32x16{};
+    for (int p = 0; p < len; p += 2) {  // lane half fh holds k = p + fh
+      const bool in = p + fh < len;
+      const int64_t pk = in ? p + fh : 0;
+      const int64_t bs = g.seg < g.K ? ((k0 + pk) / g.seg - seg0) * bfix : 0;
+      float a[MT], b[NT];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const float v = A0[AKM ? static_cast<int64_t>(ra[i]) * g.lda + pk : pk * g.lda + ra[i]];
+        a[i] = in ? v : 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const float v = B0[bs + (BKM ? static_cast<int64_t>(rb[j]) * g.ldb + pk : pk * g.ldb + rb[j])];
+        b[j] = in ? v : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+  }
+
+  // split: partial products side by side, (q, part, m, n)
+  const bool split = g.nsplit > 1;
+  float* __restrict__ Cq = split ? C + static_cast<int64_t>(blockIdx.z) * g.M * g.N : C + q * g.sc;
+  const int64_t ldc = split ? g.N : g.ldc;
+  const bool add = !split && g.accumulate;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int col = n0 + wn + j * 32 + fr;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = m0 + wm + i * 32 + 8 * (r / 4) + 4 * fh + (r & 3);
+        if (row < g.M && col < g.N) {
+          float* c = Cq + row * ldc + col;
+          *c = add ? *c + acc[i][j][r] : acc[i][j][r];
+        }
+      }
+    }
+}
+
+// C (+)= the sum of the partial products, left to right
+template <typename V>
+__global__ void __launch_bounds__(kThreads)
+gemm_reduce_kernel(GemmGeom g, const float* __restrict__ part, float* __restrict__ C) {
+  constexpr int W = sizeof(V) / sizeof(float);
+  const int64_t mn = static_cast<int64_t>(g.M) * g.N;
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * W;
+  if (i >= mn) return;
+  const int64_t q = blockIdx.y;
+  const float* p = part + q * g.nsplit * mn + i;
+  const int64_t row = i / g.N;
+  float* c = C + q * g.sc + row * g.ldc + (i - row * g.N);
+  float s[W];
+  V v = *reinterpret_cast<const V*>(p);
+#pragma unroll
+  for (int e = 0; e < W; ++e) s[e] = reinterpret_cast<const float*>(&v)[e];
+  for (int z = 1; z < g.nsplit; ++z) {
+    v = *reinterpret_cast<const V*>(p + z * mn);
+#pragma unroll
+    for (int e = 0; e < W; ++e) s[e] += reinterpret_cast<const float*>(&v)[e];
+  }
+  if (g.accumulate) {
+    v = *reinterpret_cast<const V*>(c);
+#pragma unroll
+    for (int e = 0; e < W; ++e) s[e] += reinterpret_cast<const float*>(&v)[e];
+  }
+#pragma unroll
+  for (int e = 0; e < W; ++e) reinterpret_cast<float*>(&v)[e] = s[e];
+  *reinterpret_cast<V*>(c) = v;
+}
+
+// Tile shapes: 2 workgroups on a CU (by VGPRs), 3 (by LDS).
+struct TileCfg {
+  int bm, bn, bk, occ;
+  // microseconds per step (bk of k) of a workgroup that has a CU to itself,
+  // and per step and workgroup of a CU that runs several (measured on the
+  // shapes of gemm_plan's comment)
+  float alone, shared;
+};
+constexpr TileCfg kCfg[2] = {{128, 128, 16, 2, 0.80f, 0.68f}, {64, 64, 32, 3, 0.50f, 0.46f}};
+constexpr int kCUs = 256;
+constexpr float kBytesPerUs = 4.5e6f;  // HBM, streaming
+constexpr int kMaxSplit = 24;
+
+template <int CFG, bool AKM, bool BKM>
+void launch_cfg(const GemmGeom& g, const float* A, const float* B, float* C, hipStream_t s) {
+  constexpr TileCfg c = kCfg[CFG];
+  const unsigned nt = static_cast<unsigned>((g.M + c.bm - 1) / c.bm) * static_cast<unsigned>((g.N + c.bn - 1) / c.bn);
+  hipLaunchKernelGGL((gemm_kernel<c.bm, c.bn, c.bk, c.occ, AKM, BKM>),
+                     dim3(nt, 1, static_cast<unsigned>(g.batch * g.nsplit)), dim3(kThreads), 0, s, g, A, B, C);
+}
+template <int CFG>
+void launch_layout(const GemmGeom& g, const float* A, const float* B, float* C, hipStream_t s) {
+  if (g.a_km)
+    g.b_km ? launch_cfg<CFG, true, true>(g, A, B, C, s) : launch_cfg<CFG, true, false>(g, A, B, C, s);
+  else
+    g.b_km ? launch_cfg<CFG, false, true>(g, A, B, C, s) : launch_cfg<CFG, false, false>(g, A, B, C, s);
+}
+
+}  // namespace
+
+// The tile shape and split with the least estimated time: the steps of the
+// busiest CU, writing C, and with a split the partial products (written and
+// read) and the second launch.  Measured (estimated) us on MI355X, the BLAS
+// library's time last: 6272 x 6144 x 384: 128-tiles unsplit 207 (189), 64-tiles
+// 241, library 248-290; 6272 x 384 x 6144: 128-tiles in 3 parts 187 (194),
+// unsplit 310, 8 parts 197, library 262; 196 x 1536 x 384: 64-tiles unsplit
+// 10.0 (6.3 + launch), 128-tiles 22.8, library 19.6; 196 x 384 x 768: 64-tiles
+// in 4-8 parts 10.3, unsplit 15.9, library 19.2.
+void gemm_plan(GemmGeom& g) {
+  const int want = g.nsplit;  // > 0: the caller's split
+  const float mn4 = 4.f * static_cast<float>(g.batch) * static_cast<float>(g.M) * static_cast<float>(g.N);
+  float best = __builtin_inff();
+  for (int c = 0; c < 2; ++c) {
+    const TileCfg& t = kCfg[c];
+    const float tiles = static_cast<float>(g.batch) * static_cast<float>((g.M + t.bm - 1) / t.bm) *
+                        static_cast<float>((g.N + t.bn - 1) / t.bn);
+    for (int ns = want > 0 ? want : 1; ns <= (want > 0 ? want : kMaxSplit); ++ns) {
+      // (at least 64 values of k per part; partial products of at most 1 GiB)
+      if (want == 0 && ns > 1 &&
+          (g.K / ns < 64 || mn4 * ns > 1073741824.f || static_cast<int64_t>(g.batch) * ns > 65535)) break;
+      const int kper = static_cast<int>((static_cast<int64_t>(g.K) + ns - 1) / ns + t.bk - 1) / t.bk * t.bk;
+      const float steps = static_cast<float>(kper / t.bk);
+      const float n = tiles * static_cast<float>(ns);
+      const float load = n <= kCUs * t.occ ? __builtin_ceilf(n / kCUs) : n / kCUs + 0.3f;
+      float us = steps * (load <= 1.f ? t.alone : t.shared * load) + mn4 / kBytesPerUs;
+      if (ns > 1) us += 3.f + 2.f * static_cast<float>(ns) * mn4 / kBytesPerUs;
+      if (us < best) {
+        best = us;
+        g.cfg = c;
+        g.nsplit = ns;
+        g.kper = kper;
+      }
+    }
+  }
+}
+
+int64_t gemm_partial_floats(const GemmGeom& g) {
+  return g.nsplit > 1 ? static_cast<int64_t>(g.batch) * g.nsplit * g.M * g.N : 0;
+}
+
+hipError_t launch_gemm(const GemmGeom& g, const float* A, const float* B, float* C, float* part,
+                       hipStream_t s) {
+  float* out = g.nsplit > 1 ? part : C;
+  switch (g.cfg) {
+    case 0: launch_layout<0>(g, A, B, out, s); break;
+    default: launch_layout<1>(g, A, B, out, s); break;
+  }
+  if (g.nsplit > 1) {
+    const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && g.sc % 4 == 0 &&
+                     (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
+    const int64_t n = static_cast<int64_t>(g.M) * g.N / (vec ? 4 : 1);
+    const dim3 grid(static_cast<unsigned>((n + kThreads - 1) / kThreads), static_cast<unsigned>(g.batch));
+    if (vec)
+      hipLaunchKernelGGL((gemm_reduce_kernel<float4>), grid, dim3(kThreads), 0, s, g, part, C);
+    else
+      hipLaunchKernelGGL((gemm_reduce_kernel<float>), grid, dim3(kThreads), 0, s, g, part, C);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace mvm

@@ -1,7 +1,8 @@
 """GEMM selections for the VisionMamba projections on MI355X.
 
-The block's projections (in_proj, x_proj, dt_proj, out_proj and their
-gradients) are plain fp32 GEMMs on the ROCm BLAS libraries.  PyTorch's
+The block's x_proj and dt_proj and their gradients, and the shapes of in_proj
+and out_proj that the HIP products do not take (gemm.py), are plain fp32 GEMMs
+on the ROCm BLAS libraries.  PyTorch's
 TunableOp can pick, per GEMM shape, the fastest of the rocBLAS and
 hipBLASLt solutions; ``tuning/gemm_mi355x_visionmamba2d.csv`` holds the
 picks measured on MI355X for the VisionMamba-2D training step (batch 32,

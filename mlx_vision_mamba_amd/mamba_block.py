@@ -27,8 +27,7 @@ copies.
 The direction blocks' per-direction parameters (in_proj, conv1d, x_proj,
 dt_proj, A_log, D, out_proj) are slices of one (K, ...) buffer per kind owned
 by the direction module, so the batched operands are views, not per-step
-concatenations (out_proj's (E, K*D_inner) operand is one reordering copy);
-each buffer's gradient returns to the K parameters as its K
+concatenations; each buffer's gradient returns to the K parameters as its K
 slices.  The buffers are (re)built at the first forward and whenever a
 parameter stops being its slice (after ``.to()``, or a replaced parameter).
 """
@@ -44,6 +43,7 @@ import torch.nn.functional as F
 
 from . import directions as _dirs
 from .conv import causal_conv_silu, conv_silu_backward_into, conv_silu_forward_into
+from .gemm import in_proj, out_proj
 from .norm import layer_norm
 from .scan import (check_permutation_table, get_scan_fn, mode_chunk_len, scan_fused_backward,
                    scan_fused_forward)
@@ -422,7 +422,7 @@ def _directional_forward(blocks, h, tok, scan_mode, stacks=None):
                                      *[p for ps in _params_of(blocks) for p in ps])
     W_in, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv, W_out = per
     W_in = W_in.reshape(K * 2 * din, W_in.shape[-1])                          # (K*2D, E)
-    xz = F.linear(h, W_in).view(bsz, n, K, 2 * din)                            # :165-167
+    xz = in_proj(h, W_in).view(bsz, n, K, 2 * din)                             # :165-167
     conv_w = conv_w.reshape(K, din, b0.d_conv)                                 # (K, Din, d_conv)
     # W_x (K, R+2N, Din), W_dt (K, Din, R), b_dt (K, Din), A_log (K, Din, N), Dv (K, Din)
     if tok is not None:
@@ -434,7 +434,5 @@ def _directional_forward(blocks, h, tok, scan_mode, stacks=None):
         args = [t.detach() for t in args]
     save = not detach and torch.is_grad_enabled() and any(t.requires_grad for t in args)
     y = _MambaCoreFn.apply(*args, tok, mode_chunk_len(scan_mode), save)       # :170-190
-    # (K, E, Din) -> (E, K*Din): the out_proj of the concatenated directions
-    # is their (atomic-free) sum
-    W_out = W_out.permute(1, 0, 2).reshape(W_out.shape[1], K * din)
-    return F.linear(y.reshape(bsz, n, K * din), W_out)                         # :191, :562-566
+    # one product over the concatenated directions: their (atomic-free) sum
+    return out_proj(y, W_out)                                                  # :191, :562-566

@@ -1,0 +1,153 @@
+"""GPU parity of the float32 products on the bf16 matrix units
+(include/mvm_gemm.h) against float64.
+
+Per element |got - ref| <= (6 * ceil(k / 16) + splits + 2) * 2^-23 * S with
+S = sum_p |a_p b_p|: one rounding of a partial sum (at most S, a unit of at
+most 2^-23) for each of the six MFMAs per 16 values of k, for each part of a
+split and for the addition to C; the products left out of the split are below
+2^-25 * S.  Over normal inputs the error in the 2-norm is also held to that of
+torch's float32 product (the BLAS library's float32 matrix instructions).
+"""
+
+import ctypes
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from mlx_vision_mamba_amd import _lib, gemm
+
+pytestmark = pytest.mark.gpu
+
+
+def _operand(rows, k, kmajor, batch, pad, gen):
+    """(logical (batch, rows, k) float64-free values, buffer, leading dim, batch stride)"""
+    r, c = (rows, k) if kmajor else (k, rows)
+    ld = -(-c // 4) * 4 + pad
+    buf = torch.randn(batch, r, ld, generator=gen).cuda()
+    v = buf[:, :, :c]
+    return (v if kmajor else v.transpose(1, 2)), buf, ld, r * ld
+
+
+def _run(desc, A, B, C):
+    lib = _lib.lib()
+    nbytes = _lib.check(lib.mvm_gemm_workspace_bytes(ctypes.byref(desc)))
+    ws = torch.full((max(nbytes, 1),), 255, dtype=torch.uint8, device="cuda")  # NaN if read before written
+    _lib.check(lib.mvm_gemm_f32(ctypes.byref(desc), A.data_ptr(), B.data_ptr(), C.data_ptr(), ws.data_ptr(),
+                                nbytes, torch.cuda.current_stream().cuda_stream))
+
+
+CASES = [
+    # m, n, k, batch, splits, pad
+    (1, 1, 1, 1, 0, 0), (3, 5, 7, 2, 0, 4), (64, 64, 32, 1, 0, 0), (65, 63, 33, 1, 0, 0),
+    (127, 129, 31, 1, 1, 0), (128, 128, 16, 1, 1, 0), (200, 131, 17, 3, 1, 4), (129, 257, 100, 1, 3, 0),
+    (300, 200, 1655, 1, 0, 0), (1100, 1300, 48, 1, 0, 0), (1100, 1300, 75, 1, 1, 0), (64, 72, 50, 1, 24, 0),
+    (70, 60, 40, 2, 64, 0), (5, 4, 0, 1, 0, 0), (2500, 1700, 36, 1, 2, 0),
+]
+
+
+@pytest.mark.parametrize("akm", [0, 1])
+@pytest.mark.parametrize("bkm", [0, 1])
+@pytest.mark.parametrize("m,n,k,batch,splits,pad", CASES)
+def test_product(cuda, m, n, k, batch, splits, pad, akm, bkm):
+    gen = torch.Generator().manual_seed(m * 7 + n * 3 + k)
+    a, A, lda, sa = _operand(m, max(k, 1), akm, batch, pad, gen)
+    b, B, ldb, sb = _operand(n, max(k, 1), bkm, batch, pad, gen)
+    ldc = n + 3
+    for acc in (0, 1):
+        C0 = torch.randn(batch, m, ldc, generator=gen).cuda()
+        C = C0.clone()
+        d = _lib.GemmDesc(m, n, k, batch, lda, ldb, ldc, sa, sb, m * ldc, 0, 0, akm, bkm, acc, splits)
+        _run(d, A, B, C)
+        ad, bd = a.double()[:, :, :k], b.double()[:, :, :k].transpose(1, 2).contiguous()
+        ref = ad @ bd + (C0.double()[:, :, :n] if acc else 0)
+        S = ad.abs() @ bd.abs() + (C0.double()[:, :, :n].abs() if acc else 0)
+        bound = (6 * -(-k // 16) + max(splits, 24) + 2) * 2.0 ** -23 * S
+        assert ((C.double()[:, :, :n] - ref).abs() <= bound).all()
+        assert torch.equal(C[:, :, n:], C0[:, :, n:])  # nothing outside the matrix
+        again = C0.clone()
+        _run(d, A, B, again)
+        assert torch.equal(again, C)
+
+
+@pytest.mark.parametrize("m,n,k", [(640, 768, 384), (392, 768, 3072), (1655, 200, 800), (384, 768, 6272)])
+@pytest.mark.parametrize("shift", [0.0, 1.0])
+def test_error_no_larger_than_float32(cuda, m, n, k, shift):
+    """Unit normal inputs, and inputs of one sign (shift: |x|, no cancellation)."""
+    gen = torch.Generator().manual_seed(k)
+    A, B = torch.randn(m, k, generator=gen).cuda(), torch.randn(n, k, generator=gen).cuda()
+    if shift:
+        A, B = A.abs(), B.abs()
+    C = torch.empty(m, n, device="cuda")
+    _run(_lib.GemmDesc(m, n, k, 1, k, k, n, 0, 0, 0, 0, 0, 1, 1, 0, 0), A, B, C)
+    ref = A.double() @ B.double().t().contiguous()
+    err = lambda x: ((x.double() - ref).norm() / ref.norm()).item()  # noqa: E731
+    assert err(C) <= err(F.linear(A, B)), (err(C), err(F.linear(A, B)))
+
+
+@pytest.mark.parametrize("K,D", [(3, 32), (4, 96), (2, 160)])
+def test_segments(cuda, K, D):
+    """One product over K weight matrices that lie apart."""
+    gen = torch.Generator().manual_seed(K)
+    M, E = 150, 72
+    y, W = torch.randn(M, K, D, generator=gen).cuda(), torch.randn(K, E, D, generator=gen).cuda()
+    ref = torch.einsum("mkd,ked->me", y.double().cpu(), W.double().cpu())
+    S = torch.einsum("mkd,ked->me", y.double().abs().cpu(), W.double().abs().cpu())
+    for splits in (0, 1, 2, 5):
+        C = torch.empty(M, E, device="cuda")
+        _run(_lib.GemmDesc(M, E, K * D, 1, K * D, D, E, 0, 0, 0, D, E * D, 1, 1, 0, splits), y, W, C)
+        assert ((C.double().cpu() - ref).abs() <= (6 * -(-K * D // 16) + 26) * 2.0 ** -23 * S).all()
+
+
+@pytest.mark.parametrize("akm,bkm", [(1, 1), (1, 0), (0, 0)])
+@pytest.mark.parametrize("k,splits", [(40, 1), (333, 3)])
+def test_special_values_as_float32(cuda, akm, bkm, k, splits):
+    """Infinities, NaN, values near the largest float32 and tiny inputs give
+    what float32 arithmetic gives."""
+    m, n = 140, 70
+    gen = torch.Generator().manual_seed(k)
+    a, A, lda, _ = _operand(m, k, akm, 1, 0, gen)
+    b, B, ldb, _ = _operand(n, k, bkm, 1, 0, gen)
+    a, b = a[0], b[0]
+    inf = float("inf")
+    a[3, 5], a[9, 7], a[20, 0] = inf, -inf, float("nan")
+    a[70] = 0.0
+    a[70, 1], b[:, 1] = 3.4028e38, 0.25  # rounds to infinity in bf16; the product is finite
+    a[100, 2], a[100, 3], b[11, 2], b[11, 3] = inf, inf, 1.0, -1.0
+    C = torch.empty(m, n, device="cuda")
+    d = _lib.GemmDesc(m, n, k, 1, lda, ldb, n, 0, 0, 0, 0, 0, akm, bkm, 0, splits)
+    _run(d, A, B, C)
+    ref = (a.double() @ b.double().t().contiguous()).float()
+    assert torch.equal(torch.isnan(C), torch.isnan(ref))
+    assert torch.equal(torch.isinf(C), torch.isinf(ref)) and (C[torch.isinf(C)] == ref[torch.isinf(ref)]).all()
+    ok = torch.isfinite(ref)
+    S = a.abs().nan_to_num(0, 0, 0).double() @ b.abs().double().t().contiguous()
+    assert ((C - ref).double().abs()[ok] <= ((k + 4) * 2.0 ** -23 * S)[ok]).all()
+    # inputs so small that the split's low parts underflow
+    A.copy_(torch.randn(A.shape, generator=gen) * 2.0 ** -118)
+    B.copy_(torch.randn(B.shape, generator=gen))
+    _run(d, A, B, C)
+    ref = a.double() @ b.double().t().contiguous()
+    S = a.abs().double() @ b.abs().double().t().contiguous()
+    assert ((C.double() - ref).abs() <= (k + 4) * (2.0 ** -23 * S + 2.0 ** -149)).all()
+
+
+@pytest.mark.parametrize("B,n,K,D,E", [(2, 37, 1, 24, 12), (3, 50, 4, 64, 40), (0, 5, 2, 32, 16), (1, 9, 2, 40, 20)])
+def test_projections_match_autograd(cuda, B, n, K, D, E):
+    """in_proj / out_proj (also where the kernels do not take the shape:
+    Din = 40 in two directions) against float64 autograd."""
+    gen = torch.Generator().manual_seed(1)
+    h = torch.randn(B, n, E, generator=gen).cuda().requires_grad_()
+    Wi = torch.randn(K * 2 * D, E, generator=gen).cuda().requires_grad_()
+    Wo = torch.randn(K, E, D, generator=gen).cuda().requires_grad_()
+    xz = gemm.in_proj(h, Wi)
+    out = gemm.out_proj(xz.view(B, n, K, 2 * D)[..., D:].contiguous(), Wo)
+    g = torch.randn(B, n, E, generator=gen).cuda()
+    got = [out, *torch.autograd.grad(out, (h, Wi, Wo), g)]
+    hd, wi, wo = [t.detach().double().cpu().requires_grad_() for t in (h, Wi, Wo)]
+    o64 = torch.einsum("bnkd,ked->bne", (hd @ wi.t()).view(B, n, K, 2 * D)[..., D:], wo)
+    ref = [o64, *torch.autograd.grad(o64, (hd, wi, wo), g.double().cpu())]
+    for x, r in zip(got, ref):
+        assert x.shape == r.shape
+        # two chained products of at most 6 * 60 roundings each
+        assert (x.double().cpu() - r).norm() <= 800 * 2.0 ** -24 * r.norm() + 1e-30
