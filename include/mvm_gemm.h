@@ -48,16 +48,16 @@ typedef struct mvm_gemm_desc {
   int32_t splits;      /* parts the sum over p is cut into; 0: chosen by the library */
 } mvm_gemm_desc;
 
-/* Validates a descriptor without touching the GPU.  A k-major operand needs
- * a leading dimension and a batch (and segment) stride that are multiples of
- * 4; leading dimensions are below 2^21.  MVM_ERR_UNSUPPORTED otherwise. */
+/* Validates a descriptor without touching the GPU.  From k = 32 up a k-major
+ * operand needs a leading dimension and a batch (and segment) stride that are
+ * multiples of 4; leading dimensions are below 2^21.  MVM_ERR_UNSUPPORTED otherwise. */
 int mvm_gemm_validate(const mvm_gemm_desc* desc);
 
 /* Bytes of workspace mvm_gemm_f32 needs (0 when the sum is not split). */
 int64_t mvm_gemm_workspace_bytes(const mvm_gemm_desc* desc);
 
-/* k-major operands must be 16-byte aligned, the workspace 256-byte aligned.
- * k = 0 writes zeros (accumulate: leaves C). */
+/* From k = 32 up k-major operands must be 16-byte aligned; the workspace must
+ * be 256-byte aligned.  k = 0 writes zeros (accumulate: leaves C). */
 int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, float* C,
                  void* workspace, size_t workspace_bytes, void* stream);
 

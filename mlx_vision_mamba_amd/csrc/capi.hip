@@ -786,8 +786,10 @@ int check_gemm(const mvm_gemm_desc* d) {
     return fail(MVM_ERR_INVALID_ARG, "gemm leading dimension smaller than its row");
   if (d->lda >= kGemmMaxLd || d->ldb >= kGemmMaxLd)
     return fail(MVM_ERR_UNSUPPORTED, "gemm leading dimension exceeds %lld", (long long)kGemmMaxLd - 1);
-  if ((d->a_kmajor && (d->lda % 4 || d->a_stride_batch % 4)) ||
-      (d->b_kmajor && (d->ldb % 4 || d->b_stride_batch % 4 || d->b_seg_stride % 4)))
+  // (k < 32: loaded value by value, see gemm_plan)
+  if (d->k >= 32 &&
+      ((d->a_kmajor && (d->lda % 4 || d->a_stride_batch % 4)) ||
+      (d->b_kmajor && (d->ldb % 4 || d->b_stride_batch % 4 || d->b_seg_stride % 4))))
     return fail(MVM_ERR_UNSUPPORTED, "a k-major gemm operand needs strides that are multiples of 4");
   if (!no_overlap({{d->batch, d->c_stride_batch}, {d->m, d->ldc}, {d->n, 1}}))
     return fail(MVM_ERR_INVALID_ARG, "gemm C strides overlap");
@@ -839,7 +841,8 @@ int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, floa
   if (rc != MVM_OK) return rc;
   if (g.M == 0 || g.N == 0 || g.batch == 0 || (g.K == 0 && g.accumulate)) return ok();
   if (!C || (g.K > 0 && (!A || !B))) return fail(MVM_ERR_INVALID_ARG, "mvm_gemm_f32: NULL pointer");
-  if ((g.a_km && (reinterpret_cast<uintptr_t>(A) & 15u)) || (g.b_km && (reinterpret_cast<uintptr_t>(B) & 15u)))
+  if (g.K >= 32 &&
+      ((g.a_km && (reinterpret_cast<uintptr_t>(A) & 15u)) || (g.b_km && (reinterpret_cast<uintptr_t>(B) & 15u))))
     return fail(MVM_ERR_INVALID_ARG, "mvm_gemm_f32: a k-major operand must be 16-byte aligned");
   const size_t need = align_up(sizeof(float) * mvm::gemm_partial_floats(g));
   if (need > 0) {

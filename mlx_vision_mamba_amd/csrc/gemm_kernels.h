@@ -21,7 +21,8 @@ struct GemmGeom {
   int32_t nsplit, kper;  // the sum over k in nsplit parts of kper
 };
 
-// picks the tile shape and (when nsplit is 0) the split of k
+// picks the tile shape and (when nsplit is 0) the split of k; below 32 values
+// of k no operand is loaded in vectors, so any alignment will do
 void gemm_plan(GemmGeom& g);
 // float32 elements of the partial-product buffer (0 without a split)
 int64_t gemm_partial_floats(const GemmGeom& g);

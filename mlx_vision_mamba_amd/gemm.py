@@ -1,5 +1,5 @@
-"""The block's in_proj and out_proj as float32 products on the bf16 matrix
-units (HIP kernels behind include/mvm_gemm.h).
+"""The block's projections as float32 products on the bf16 matrix units (HIP
+kernels behind include/mvm_gemm.h).
 
 Replaces the reference's ``nn.Linear`` in_proj and out_proj
 (mamba_block.py:125, :153, :165, :191) for all K directions of a block:
@@ -9,7 +9,9 @@ Replaces the reference's ``nn.Linear`` in_proj and out_proj
 
 The out_proj reads the K stacked weight matrices where they lie, as one
 product over K*Din, and its weight gradient comes out in the same (K, E, Din)
-layout, so no reordered copy of either is made.
+layout, so no reordered copy of either is made.  ``batched`` runs the
+direction-batched products of x_proj and dt_proj (:137-140, :174-180) and their
+gradients.
 """
 
 from __future__ import annotations
@@ -29,8 +31,10 @@ def _aligned(t):
     return t.data_ptr() % 16 == 0
 
 
-def _launch(A, B, C, m, n, k, lda, ldb, ldc, a_km, b_km, batch=1, sa=0, sb=0, sc=0, seg=0, seg_stride=0):
-    d = _lib.GemmDesc(m, n, k, batch, lda, ldb, ldc, sa, sb, sc, seg, seg_stride, a_km, b_km, 0, 0)
+def _launch(A, B, C, m, n, k, lda, ldb, ldc, a_km, b_km, batch=1, sa=0, sb=0, sc=0, seg=0, seg_stride=0,
+            accumulate=False):
+    d = _lib.GemmDesc(m, n, k, batch, lda, ldb, ldc, sa, sb, sc, seg, seg_stride, a_km, b_km,
+                      int(accumulate), 0)
     lib = _lib.lib()
     dev = C.device
     with torch.cuda.device(dev):
@@ -128,3 +132,39 @@ def out_proj(y, W):
         return _OutProjFn.apply(y, W)
     # one product over the concatenated directions (a reordered copy of W)
     return F.linear(y.reshape(*y.shape[:-2], K * D), W.permute(1, 0, 2).reshape(E, K * D))
+
+
+# batch x rows from which dt_proj's two products over the rows (the delta_raw
+# and its gradient's) are left to the BLAS library: they stream 77 MB at 4 x
+# 6272 rows of 768 channels, with almost no arithmetic, and the library's picks
+# take 25.6 and 22.3 us there, the kernels here 31.4 and 27.3; at 8 x 1024 rows
+# it is 21 and 20 us against 12.1 and 13.7.
+STREAM_ROWS = 16384
+
+
+def _rowmajor(t):
+    """Whether (batch, rows, cols) t has contiguous columns and 16-byte rows."""
+    return (t.stride(2) == 1 and t.stride(1) % 4 == 0 and t.stride(0) % 4 == 0 and _aligned(t)
+            and t.stride(1) < 1 << 21)
+
+
+def batched(A, B, out=None, ta=False, tb=False, accumulate=False, stream=False):
+    """out[q] (+)= op(A[q]) @ op(B[q]) for float32 (batch, rows, cols) views
+    with contiguous columns; ta / tb transpose an operand.  An operand whose
+    summed index is its contiguous one (A without ta, B with tb) needs 16-byte
+    rows from 32 summed values up, and out columns that are contiguous; where
+    the kernels do not take the operands, and for a ``stream`` product of many
+    rows, torch computes it."""
+    Av, Bv = (A.transpose(1, 2) if ta else A), (B.transpose(1, 2) if tb else B)
+    q, m, k = Av.shape
+    n = Bv.shape[2]
+    if out is None:
+        out = torch.empty((q, m, n), dtype=torch.float32, device=A.device)
+    ok = (A.stride(2) == 1 and B.stride(2) == 1 and max(A.stride(1), B.stride(1)) < 1 << 21
+          and (k < 32 or ((ta or _rowmajor(A)) and (not tb or _rowmajor(B))))
+          and not (stream and q * m > STREAM_ROWS))
+    if ok:
+        _launch(A, B, out, m, n, k, A.stride(1), B.stride(1), out.stride(1), int(not ta), int(tb),
+                batch=q, sa=A.stride(0), sb=B.stride(0), sc=out.stride(0), accumulate=accumulate)
+        return out
+    return out.baddbmm_(Av, Bv) if accumulate else torch.bmm(Av, Bv, out=out)

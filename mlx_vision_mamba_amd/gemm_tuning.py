@@ -1,8 +1,7 @@
 """GEMM selections for the VisionMamba projections on MI355X.
 
-The block's x_proj and dt_proj and their gradients, and the shapes of in_proj
-and out_proj that the HIP products do not take (gemm.py), are plain fp32 GEMMs
-on the ROCm BLAS libraries.  PyTorch's
+dt_proj's products over many rows, and projections of shapes that the HIP
+products do not take (gemm.py), are plain fp32 GEMMs on the ROCm BLAS libraries.  PyTorch's
 TunableOp can pick, per GEMM shape, the fastest of the rocBLAS and
 hipBLASLt solutions; ``tuning/gemm_mi355x_visionmamba2d.csv`` holds the
 picks measured on MI355X for the VisionMamba-2D training step (batch 32,

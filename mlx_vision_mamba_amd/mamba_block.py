@@ -43,7 +43,7 @@ import torch.nn.functional as F
 
 from . import directions as _dirs
 from .conv import causal_conv_silu, conv_silu_backward_into, conv_silu_forward_into
-from .gemm import in_proj, out_proj
+from .gemm import batched, in_proj, out_proj
 from .norm import layer_norm
 from .scan import (check_permutation_table, get_scan_fn, mode_chunk_len, scan_fused_backward,
                    scan_fused_forward)
@@ -301,10 +301,11 @@ class _MambaCoreFn(torch.autograd.Function):
         xb, z = xz[..., :din], xz[..., din:]
         xc = torch.empty(K, bsz * n, din, dtype=torch.float32, device=dev)
         conv_silu_forward_into(xb, conv_w, conv_b, _bnkd(xc, bsz, n), tok)       # :170-171
-        # float32 operands: the GEMMs take the weights' transposed views as they are
-        dbc = torch.bmm(xc, W_x.transpose(1, 2))                                   # :174
-        dt = dbc[..., :R]
-        delta_raw = torch.bmm(dt, W_dt.transpose(1, 2))                            # :180
+        # rows of a multiple of 4 values: 16-byte rows for the products that read them
+        P = R + 2 * ns
+        dbc = torch.empty(K, bsz * n, -(-P // 4) * 4, dtype=torch.float32, device=dev)[..., :P]
+        batched(xc, W_x, out=dbc, tb=True)                                         # :174
+        delta_raw = batched(dbc[..., :R], W_dt, tb=True, stream=True)              # :180
         bc = _bnkd(dbc, bsz, n)
         # save: checkpoints and y_raw are kept for the backward (training);
         # off for the forward-only mode and under no_grad / inference_mode
@@ -328,7 +329,7 @@ class _MambaCoreFn(torch.autograd.Function):
         dev = xz.device
         xb, z = xz[..., :din], xz[..., din:]
         dxz = torch.empty(xz.shape, dtype=torch.float32, device=dev)
-        d_dbc = torch.empty_like(dbc)
+        d_dbc = torch.empty(K, bsz * n, dbc.stride(1), dtype=torch.float32, device=dev)[..., :dbc.shape[2]]
         du = torch.empty_like(xc)
         ddelta_raw = torch.empty_like(delta_raw)
         bc, dbc_v = _bnkd(dbc, bsz, n), _bnkd(d_dbc, bsz, n)
@@ -337,32 +338,18 @@ class _MambaCoreFn(torch.autograd.Function):
             bc[..., R + ns:], Dv, z, y_raw, ckpt, dy, tok, ctx.chunk_len,
             du=_bnkd(du, bsz, n), ddelta_raw=_bnkd(ddelta_raw, bsz, n),
             dB=dbc_v[..., R:R + ns], dC=dbc_v[..., R + ns:], dz=dxz[..., din:], a_is_log=True)
-        # dt_proj: delta_raw = dt @ W_dt^T; the GEMM writes the first R columns
-        # of d_dbc in place (row stride R + 2N is a valid leading dimension)
-        torch.bmm(ddelta_raw, W_dt, out=d_dbc[..., :R])
-        dW_dt = torch.bmm(ddelta_raw.transpose(1, 2), dbc[..., :R])
-        # x_proj: dbc = xc @ W_x^T; the scan's du joins through the GEMM's beta
-        # (in place: du is this backward's own buffer, so no copy of it is made)
-        dxc = du.baddbmm_(d_dbc, W_x)
-        dW_x = _tn_split_rows(d_dbc, xc)
+        # dt_proj: delta_raw = dt @ W_dt^T; the product writes the first R
+        # columns of d_dbc in place
+        batched(ddelta_raw, W_dt, out=d_dbc[..., :R], stream=True)
+        dW_dt = batched(ddelta_raw, dbc[..., :R], ta=True)
+        # x_proj: dbc = xc @ W_x^T; its input gradient is added to the scan's
+        # du (this backward's own buffer)
+        dxc = batched(d_dbc, W_x, out=du, accumulate=True)
+        dW_x = batched(d_dbc, xc, ta=True)
         # conv + SiLU: dx lands in the first half of dxz
         dconv_w, dconv_b = conv_silu_backward_into(xb, conv_w, conv_b, _bnkd(dxc, bsz, n),
                                                    dxz[..., :din], tok)
         return dxz, dconv_w, dconv_b, dW_x, dW_dt, db_dt, dA_log, dDv, None, None, None
-
-
-def _tn_split_rows(a, b, splits=8):
-    """a^T @ b per direction for a (K, M, P) and b (K, M, Q) with a long row
-    reduction (M = B*N) and small outputs: the rows are split into ``splits``
-    chunks, one batched GEMM over K*splits computes the partial products and
-    they are summed in a fixed order (deterministic).  The split keeps enough
-    workgroups in flight to stream b from HBM."""
-    K, M, P = a.shape
-    if M % splits or M // splits < 256:
-        return torch.bmm(a.transpose(1, 2), b)
-    m = M // splits
-    part = torch.bmm(a.reshape(K * splits, m, P).transpose(1, 2), b.reshape(K * splits, m, -1))
-    return part.view(K, splits, P, -1).sum(1)
 
 
 def _custom_scan(blk):

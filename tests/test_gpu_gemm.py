@@ -151,3 +151,32 @@ def test_projections_match_autograd(cuda, B, n, K, D, E):
         assert x.shape == r.shape
         # two chained products of at most 6 * 60 roundings each
         assert (x.double().cpu() - r).norm() <= 800 * 2.0 ** -24 * r.norm() + 1e-30
+
+
+@pytest.mark.parametrize("q,m,k,n", [(1, 196, 24, 96), (2, 331, 13, 40), (2, 90, 29, 33), (1, 70, 50, 30),
+                                     (3, 64, 32, 24), (2, 9000, 24, 16), (2, 9000, 16, 24)])
+def test_batched_matches_float64(cuda, q, m, k, n):
+    """The direction-batched products in the forms of x_proj and dt_proj:
+    plain and transposed operands, column slices of a wider buffer (rows of a
+    multiple of 4 and not), accumulation, and the streamed ones."""
+    gen = torch.Generator().manual_seed(m + k)
+    rn = lambda *s: torch.randn(*s, generator=gen).cuda()  # noqa: E731
+    for pad in (0, 3, 4):
+        wide = rn(q, m, k + pad)
+        a, at = wide[..., :k], rn(q, k, m + pad)[..., :m]
+        b, bt = rn(q, k, n), rn(q, n, k + pad)[..., :k]
+        for A, ta in ((a, False), (at, True)):
+            for B, tb in ((b, False), (bt, True)):
+                for stream in (False, True):
+                    Ad = (A.transpose(1, 2) if ta else A).double()
+                    Bd = (B.transpose(1, 2) if tb else B).contiguous().double()
+                    ref, S = Ad @ Bd, Ad.abs() @ Bd.abs()
+                    bound = (6 * -(-k // 16) + 26) * 2.0 ** -23
+                    got = gemm.batched(A, B, ta=ta, tb=tb, stream=stream)
+                    assert ((got.double() - ref).abs() <= bound * S).all()
+                    out = rn(q, m, n + pad)
+                    keep = out.clone()
+                    gemm.batched(A, B, out=out[..., :n], ta=ta, tb=tb, accumulate=True)
+                    r2, S2 = ref + keep[..., :n].double(), S + keep[..., :n].double().abs()
+                    assert ((out[..., :n].double() - r2).abs() <= bound * S2).all()
+                    assert torch.equal(out[..., n:], keep[..., n:])
