@@ -35,8 +35,8 @@
 // memory (held in registers two steps ahead) into double-buffered LDS; each
 // fragment read from LDS then feeds six MFMAs.  A thread holds 8 consecutive
 // k of one row, whichever way the operand lies in memory, so both layouts
-// arrive in LDS the same way.  The 16-byte chunks of a row are swapped by a
-// bit of the row so that neither the writes nor the fragment reads of 8
+// arrive in LDS the same way.  The 16-byte chunks of a row are permuted by
+// bits of the row so that neither the writes nor the fragment reads of 16
 // neighbouring lanes share a bank.
 // Bound: with the MFMAs alone the loop runs at 230-240 TFLOP/s; the
 // split's VALU work (11 instructions per pair of values), the LDS traffic and
@@ -138,10 +138,11 @@ struct Operand {
       }
     }
   }
-  // LDS position of a row's chunk: 8 neighbouring rows at one chunk cover
-  // all the 16-byte columns of 128 bytes
+  // LDS position of a row's chunk: at one chunk, 16 neighbouring rows cover
+  // all the 16-byte columns of 256 bytes (as the reads are served) and 8 rows
+  // those of 128 bytes (the writes)
   __device__ static __forceinline__ int swz(int r, int c) {
-    return BK == 16 ? (c ^ ((r >> 2) & 1)) * 8 : (c ^ ((r >> 1) & 3)) * 8;
+    return BK == 16 ? (c ^ (((r >> 2) ^ (r >> 3)) & 1)) * 8 : (c ^ (((r >> 1) ^ (r >> 3)) & 3)) * 8;
   }
   __device__ __forceinline__ void store(uint16_t (*lds)[ROWS][BK], const float (&v)[kItems][8]) const {
 #pragma unroll
