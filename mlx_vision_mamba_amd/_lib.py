@@ -173,6 +173,24 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The C++ host module over the library (csrc/torch_ext.cpp; ImportError
+    if it has not been built)."""
+    global _native
+    if _native is None:
+        lib()  # checks the ABI version of the library it links
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise ImportError("mlx_vision_mamba_amd/_native.so is missing or does not load: build it with "
+                              "`python -m mlx_vision_mamba_amd.build`") from e
+        _native = mod
+    return _native
+
+
 def last_error() -> str:
     return lib().mvm_last_error().decode()
 

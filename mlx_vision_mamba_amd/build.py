@@ -1,4 +1,6 @@
-"""Builds libmvm_scan.so (the HIP kernels + C ABI) in-tree for gfx950.
+"""Builds libmvm_scan.so (the HIP kernels + C ABI) in-tree for gfx950, and
+_native.so (the C++ host path over it, csrc/torch_ext.cpp) against the
+installed torch.
 
     python -m mlx_vision_mamba_amd.build
 
@@ -23,6 +25,7 @@ CSRC = os.path.join(PKG, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 LIB = os.path.join(PKG, "libmvm_scan.so")
 SOURCES = ["capi.hip", "scan_fwd.hip", "scan_bwd.hip", "conv.hip", "layernorm.hip", "gemm.hip", "optim.hip"]
+NATIVE = os.path.join(PKG, "_native.so")
 ARCH = "gfx950"
 
 
@@ -70,7 +73,32 @@ def build(verbose: bool = False, extra=()) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
+    build_native()
     return LIB
+
+
+def build_native() -> str:
+    """Compile csrc/torch_ext.cpp (host code only) into NATIVE; returns its path."""
+    import sysconfig
+
+    import torch
+    tdir = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    inc = [os.path.join(tdir, "include"), os.path.join(tdir, "include", "torch", "csrc", "api", "include"),
+           "/opt/rocm/include" if os.path.isdir("/opt/rocm/include") else os.path.join(rocm, "include"),
+           sysconfig.get_paths()["include"]]
+    tmp = NATIVE + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_native",
+           *[a for d in inc for a in ("-isystem", d)], f"-I{INCLUDE}",
+           os.path.join(CSRC, "torch_ext.cpp"), "-o", tmp,
+           f"-L{os.path.join(tdir, 'lib')}", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+           "-ltorch_python", f"-L{PKG}", "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for torch_ext.cpp:\n{res.stderr}")
+    os.replace(tmp, NATIVE)
+    return NATIVE
 
 
 if __name__ == "__main__":

@@ -41,12 +41,11 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from . import directions as _dirs
-from .conv import causal_conv_silu, conv_silu_backward_into, conv_silu_forward_into
-from .gemm import batched, in_proj, out_proj
+from .conv import causal_conv_silu
 from .norm import layer_norm
-from .scan import (check_permutation_table, get_scan_fn, mode_chunk_len, scan_fused_backward,
-                   scan_fused_forward)
+from .scan import _resolve_chunk, check_permutation_table, get_scan_fn, mode_chunk_len
 
 
 def _dt_bias_init(d_inner: int, dt_min: float = 1e-3, dt_max: float = 1e-1) -> torch.Tensor:
@@ -132,8 +131,7 @@ class BidirectionalMambaBlock(nn.Module):
         blocks = [self.forward_mamba, self.backward_mamba]
         if any(_custom_scan(b) for b in blocks):
             return xr + _per_direction_forward(blocks, h, tok)
-        return xr + _directional_forward(blocks, h, tok, self.scan_mode,
-                                         _direction_stacks(self, blocks))
+        return xr + _directional_forward(blocks, h, tok, self.scan_mode, self, blocks)
 
 
 class MultiDirectionalMambaBlock(nn.Module):
@@ -176,8 +174,8 @@ class MultiDirectionalMambaBlock(nn.Module):
             blocks = list(self.mamba_blocks)
         if any(_custom_scan(b) for b in blocks):
             return xr + _per_direction_forward(blocks, h, tok)
-        stacks = _direction_stacks(self, list(self.mamba_blocks))
-        return xr + _directional_forward(blocks, h, tok, self.scan_mode, stacks)  # :562-566
+        return xr + _directional_forward(blocks, h, tok, self.scan_mode, self,
+                                         list(self.mamba_blocks))                # :562-566
 
 
 # per-direction parameters stored as slices of one (K, ...) buffer per kind
@@ -224,44 +222,31 @@ def _direction_stacks(owner, blocks):
     compares each parameter's data pointer, shape and dtype with those its
     slice was given (the buffers are held here, so their memory is never
     reused while the pointers are compared)."""
-    params = _params_of(blocks)
-    cache = owner.__dict__.get("_param_stacks")
-    if cache is not None:
-        bufs, expect = cache
-        flat = [p for ps in params for p in ps]
-        if len(flat) == len(expect) and all(
-                p.data_ptr() == ptr and p.dtype is dt and p.shape == shp
-                for p, (ptr, dt, shp) in zip(flat, expect)):
-            return bufs
+    return _stacks_of(owner, _params_of(blocks))
+
+
+def _stacks_of(owner, params):
+    flat = [p for ps in params for p in ps]
+    bufs = owner.__dict__.get("_param_stacks")
+    if bufs is not None and _lib.native().stacks_match(bufs, flat):
+        return bufs
     with torch.no_grad():
         bufs = [torch.stack([p.detach() for p in ps], 0) for ps in params]
         for buf, ps in zip(bufs, params):
             for k, p in enumerate(ps):
                 p.data = buf[k]
-    expect = [(p.data_ptr(), p.dtype, p.shape) for ps in params for p in ps]
-    owner.__dict__["_param_stacks"] = (bufs, expect)
+    owner.__dict__["_param_stacks"] = bufs
     return bufs
 
 
-class _DirectionParams(torch.autograd.Function):
+class _DirectionParams:
     """(buffers..., parameters...) -> the buffers, differentiable w.r.t. the
-    parameters that are their slices: the backward hands each buffer's
-    gradient to its K parameters as K contiguous slices (a gradient that
-    arrives strided, as out_proj's does, is made contiguous once, so the
-    parameters take their slices without a copy each)."""
+    parameters that are their slices (csrc/torch_ext.cpp): the backward hands
+    each buffer's gradient to its K parameters as K contiguous slices."""
 
     @staticmethod
-    def forward(ctx, nbuf, *tensors):
-        ctx.nbuf = nbuf
-        ctx.K = tensors[0].shape[0]
-        return tuple(t.view_as(t) for t in tensors[:nbuf])
-
-    @staticmethod
-    def backward(ctx, *grads):
-        out = [None] * (1 + ctx.nbuf)
-        for g in grads:
-            out += list(g.contiguous().unbind(0)) if g is not None else [None] * ctx.K
-        return tuple(out)
+    def apply(nbuf, *tensors):
+        return tuple(_lib.native().direction_params(list(tensors[:nbuf]), list(tensors[nbuf:])))
 
 
 def _cached_table(cache, K, n, grid, device):
@@ -271,85 +256,6 @@ def _cached_table(cache, K, n, grid, device):
         check_permutation_table(table)
         cache[key] = table
     return cache[key]
-
-
-def _bnkd(t_kbnd, bsz, n):
-    """(B, N, K, X) view of a direction-major (K, B*N, X) tensor."""
-    K, _, X = t_kbnd.shape
-    return t_kbnd.view(K, bsz, n, X).permute(1, 2, 0, 3)
-
-
-class _MambaCoreFn(torch.autograd.Function):
-    """xz (B, N, K, 2*D_inner) from in_proj -> gated scan output (B, N, K, D_inner).
-
-    Forward (mamba_block.py:166-190, all K directions at once):
-      xc    = silu(causal depthwise conv(x) + conv_b)      along each scan order
-      dbc   = x_proj(xc)                                   (K, B*N, R + 2N)
-      delta = softplus(dt_proj(dbc[:R]) + dt_bias)         inside the scan
-      y     = scan(xc, delta, -exp(A_log), B, C, D) * silu(z)
-    The scan kernels take A_log and form A = -exp(A_log) themselves; their
-    dA output is the gradient of A_log.
-    """
-
-    @staticmethod
-    def forward(ctx, xz, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv, tok, chunk_len, save):
-        bsz, n, K, d2 = xz.shape
-        din = d2 // 2
-        R = W_dt.shape[2]
-        ns = A_log.shape[2]
-        dev = xz.device
-        xb, z = xz[..., :din], xz[..., din:]
-        xc = torch.empty(K, bsz * n, din, dtype=torch.float32, device=dev)
-        conv_silu_forward_into(xb, conv_w, conv_b, _bnkd(xc, bsz, n), tok)       # :170-171
-        # rows of a multiple of 4 values: 16-byte rows for the products that read them
-        P = R + 2 * ns
-        dbc = torch.empty(K, bsz * n, -(-P // 4) * 4, dtype=torch.float32, device=dev)[..., :P]
-        batched(xc, W_x, out=dbc, tb=True)                                         # :174
-        delta_raw = batched(dbc[..., :R], W_dt, tb=True, stream=True)              # :180
-        bc = _bnkd(dbc, bsz, n)
-        # save: checkpoints and y_raw are kept for the backward (training);
-        # off for the forward-only mode and under no_grad / inference_mode
-        y, y_raw, ckpt = scan_fused_forward(_bnkd(xc, bsz, n), _bnkd(delta_raw, bsz, n), b_dt, A_log,
-                                            bc[..., R:R + ns], bc[..., R + ns:], Dv, z, tok,
-                                            chunk_len, save=save, a_is_log=True)   # :181-190
-        if save:
-            ctx.save_for_backward(xz, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv, tok, xc, dbc,
-                                  delta_raw, y_raw, ckpt)
-            ctx.chunk_len = chunk_len
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        (xz, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv, tok, xc, dbc, delta_raw, y_raw,
-         ckpt) = ctx.saved_tensors
-        bsz, n, K, d2 = xz.shape
-        din = d2 // 2
-        R = W_dt.shape[2]
-        ns = A_log.shape[2]
-        dev = xz.device
-        xb, z = xz[..., :din], xz[..., din:]
-        dxz = torch.empty(xz.shape, dtype=torch.float32, device=dev)
-        d_dbc = torch.empty(K, bsz * n, dbc.stride(1), dtype=torch.float32, device=dev)[..., :dbc.shape[2]]
-        du = torch.empty_like(xc)
-        ddelta_raw = torch.empty_like(delta_raw)
-        bc, dbc_v = _bnkd(dbc, bsz, n), _bnkd(d_dbc, bsz, n)
-        _, _, db_dt, dA_log, _, _, dDv, _ = scan_fused_backward(
-            _bnkd(xc, bsz, n), _bnkd(delta_raw, bsz, n), b_dt, A_log, bc[..., R:R + ns],
-            bc[..., R + ns:], Dv, z, y_raw, ckpt, dy, tok, ctx.chunk_len,
-            du=_bnkd(du, bsz, n), ddelta_raw=_bnkd(ddelta_raw, bsz, n),
-            dB=dbc_v[..., R:R + ns], dC=dbc_v[..., R + ns:], dz=dxz[..., din:], a_is_log=True)
-        # dt_proj: delta_raw = dt @ W_dt^T; the product writes the first R
-        # columns of d_dbc in place
-        batched(ddelta_raw, W_dt, out=d_dbc[..., :R], stream=True)
-        dW_dt = batched(ddelta_raw, dbc[..., :R], ta=True)
-        # x_proj: dbc = xc @ W_x^T; its input gradient is added to the scan's
-        # du (this backward's own buffer)
-        dxc = batched(d_dbc, W_x, out=du, accumulate=True)
-        dW_x = batched(d_dbc, xc, ta=True)
-        # conv + SiLU: dx lands in the first half of dxz
-        dconv_w, dconv_b = conv_silu_backward_into(xb, conv_w, conv_b, _bnkd(dxc, bsz, n),
-                                                   dxz[..., :din], tok)
-        return dxz, dconv_w, dconv_b, dW_x, dW_dt, db_dt, dA_log, dDv, None, None, None
 
 
 def _custom_scan(blk):
@@ -393,33 +299,19 @@ def _per_direction_forward(blocks, h, tok):
     return y
 
 
-def _directional_forward(blocks, h, tok, scan_mode, stacks=None):
+def _directional_forward(blocks, h, tok, scan_mode, owner=None, stacked=None):
     """Run len(blocks) MambaBlocks on one (B, N, E) input, block k scanning
-    in the order of tok[k], and return the sum of their outputs.  ``stacks``:
-    the buffers of _direction_stacks whose leading slices hold the blocks'
-    parameters (None: a single block, whose parameters are used as views)."""
+    in the order of tok[k], and return the sum of their outputs.  The
+    parameters of ``stacked`` (all direction blocks of ``owner``, of which
+    ``blocks`` are the first) are slices of one buffer per kind; without an
+    owner there is one block, whose parameters are used as they are."""
     K = len(blocks)
-    b0 = blocks[0]
-    bsz, n, _ = h.shape
-    din, ns, R = b0.d_inner, b0.d_state, b0.dt_rank
-    if stacks is None:
-        per = [ps[0].unsqueeze(0) for ps in _params_of([b0])]
+    if owner is None:
+        params, stacks = _params_of(blocks), []
     else:
-        per = _DirectionParams.apply(len(stacks), *[buf[:K] for buf in stacks],
-                                     *[p for ps in _params_of(blocks) for p in ps])
-    W_in, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv, W_out = per
-    W_in = W_in.reshape(K * 2 * din, W_in.shape[-1])                          # (K*2D, E)
-    xz = in_proj(h, W_in).view(bsz, n, K, 2 * din)                             # :165-167
-    conv_w = conv_w.reshape(K, din, b0.d_conv)                                 # (K, Din, d_conv)
-    # W_x (K, R+2N, Din), W_dt (K, Din, R), b_dt (K, Din), A_log (K, Din, N), Dv (K, Din)
-    if tok is not None:
-        tok = tok.to(h.device).contiguous()
+        params = _params_of(stacked)
+        stacks = _stacks_of(owner, params)
+    flat = [p for ps in params for p in ps[:K]]
+    chunk_len = _resolve_chunk(h.shape[1], mode_chunk_len(scan_mode))
     # the reference's "metal" mode is inference only (mamba_metal.py:230)
-    detach = scan_mode == "metal"
-    args = [t.float() for t in (xz, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv)]
-    if detach:
-        args = [t.detach() for t in args]
-    save = not detach and torch.is_grad_enabled() and any(t.requires_grad for t in args)
-    y = _MambaCoreFn.apply(*args, tok, mode_chunk_len(scan_mode), save)       # :170-190
-    # one product over the concatenated directions: their (atomic-free) sum
-    return out_proj(y, W_out)                                                  # :191, :562-566
+    return _lib.native().directional(h, flat, stacks, K, tok, chunk_len, scan_mode == "metal")

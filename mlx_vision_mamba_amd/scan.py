@@ -1,4 +1,5 @@
-"""Selective scan on MI355X: autograd Functions over the HIP C ABI.
+"""Selective scan on MI355X: the scan entry points over the HIP C ABI (their
+autograd Function and launches are in csrc/torch_ext.cpp).
 
 Drop-in for the reference's scan entry points (paths relative to the
 reference repository root):
@@ -44,6 +45,10 @@ def set_scan_timing(records):
     """Start (pass a list) or stop (pass None) recording scan launches."""
     global _timing
     _timing = records
+    if records is None:
+        _lib.native().set_timer(None, None)
+    else:
+        _lib.native().set_timer(_timer_start, _timer_stop)
 
 
 def _timer_start():
@@ -58,11 +63,12 @@ def _timer_start():
     return rec, ev
 
 
-def _timer_stop(rec, ev0, kind, nbytes_fn):
+def _timer_stop(started, kind, nbytes):
+    rec, ev0 = started
     if rec is not None:
         ev1 = torch.cuda.Event(enable_timing=True)
         ev1.record()
-        rec.append((kind, ev0, ev1, nbytes_fn()))
+        rec.append((kind, ev0, ev1, nbytes))
 
 
 def algorithmic_bytes(bsz, L, D, N, in_size, out_size, ndir=1):
@@ -90,15 +96,6 @@ def algorithmic_bytes_fused(bsz, L, D, N, ndir=1, gate=True, bias=True):
         fwd += ndir * D * 4
         vjp += ndir * D * 8
     return fwd, vjp
-
-
-def _record(kind, u, Bm, in_dt, out_dt):
-    bsz, L, K, D = u.shape
-    fwd, vjp = algorithmic_bytes(bsz * K, L, D, Bm.shape[-1], _SIZE[in_dt], _SIZE[out_dt], K)
-    return fwd if kind == "fwd" else vjp
-
-
-_SIZE = {torch.float32: 4, torch.bfloat16: 2}
 
 
 def _stream_ptr(device) -> int:
@@ -141,145 +138,25 @@ def _resolve_chunk(L, chunk_len):
     return int(chunk_len)
 
 
-def _prepare(u, delta, A, Bm, Cm, Dv):
-    """Canonicalise dtypes / layouts; shapes are (B,L,K,D), (K,D,N), (B,L,K,N), (K,D)."""
-    if u.dim() != 4 or delta.shape != u.shape:
-        raise ValueError(f"u and delta must be (B, L, K, D) of equal shape; got {tuple(u.shape)}, "
-                         f"{tuple(delta.shape)}")
-    bsz, L, K, D = u.shape
-    if A.dim() != 3 or A.shape[0] != K or A.shape[1] != D:
-        raise ValueError(f"A must be (K={K}, D={D}, N); got {tuple(A.shape)}")
-    N = A.shape[2]
-    if N < 1 or N > _lib.MVM_MAX_DSTATE:
-        raise ValueError(f"d_state={N} unsupported (1..{_lib.MVM_MAX_DSTATE})")
-    if Bm.shape != (bsz, L, K, N) or Cm.shape != (bsz, L, K, N):
-        raise ValueError(f"B and C must be {(bsz, L, K, N)}; got {tuple(Bm.shape)}, {tuple(Cm.shape)}")
-    if Dv.shape != (K, D):
-        raise ValueError(f"D must be {(K, D)}; got {tuple(Dv.shape)}")
-    _check_device(u, delta, A, Bm, Cm, Dv)
-    in_dt = torch.bfloat16 if all(t.dtype == torch.bfloat16 for t in (u, Bm, Cm)) else torch.float32
-    u = u.to(in_dt).contiguous()
-    Bm = Bm.to(in_dt)
-    Cm = Cm.to(in_dt)
-    # B / C views (e.g. column slices of a projection output) are kept when
-    # they share strides and no two elements overlap; a broadcast (stride 0)
-    # layout is copied, so that dB / dC get one element per (b, t, k, n)
-    if not (Bm.stride() == Cm.stride() and Bm.stride(-1) == 1 and min(Bm.stride()) >= 0
-            and _no_overlap(Bm)):
-        Bm, Cm = Bm.contiguous(), Cm.contiguous()
-    delta = delta.to(torch.float32).contiguous()
-    A = A.to(torch.float32).contiguous()
-    Dv = Dv.to(torch.float32).contiguous()
-    return u, delta, A, Bm, Cm, Dv, in_dt
-
-
 def scan_forward(u, delta, A, Bm, Cm, Dv, tok=None, chunk_len=0, out_dtype=None, save_ckpt=False):
     """Raw forward launch (no autograd).  Returns (y, ckpt or None).
 
     Shapes: u, delta (B,L,K,D); A (K,D,N); Bm, Cm (B,L,K,N); Dv (K,D);
     tok (K,L) int32 on the same device or None.
     """
-    u, delta, A, Bm, Cm, Dv, in_dt = _prepare(u, delta, A, Bm, Cm, Dv)
-    out_dt = out_dtype or in_dt
-    L = u.shape[1]
-    desc = _make_desc(u, Bm, in_dt, out_dt, tok, _resolve_chunk(L, chunk_len))
-    lib = _lib.lib()
-    dev = u.device
-    with torch.cuda.device(dev):
-        y = torch.empty(u.shape, dtype=out_dt, device=dev)
-        ckpt = None
-        if save_ckpt:
-            ckpt = torch.empty(_lib.check(lib.mvm_scan_ckpt_elems(ctypes.byref(desc))),
-                               dtype=torch.float32, device=dev)
-        nbytes = _lib.check(lib.mvm_scan_workspace_bytes(ctypes.byref(desc), 0))
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-        rec, ev0 = _timer_start()
-        _lib.check(lib.mvm_scan_fwd(ctypes.byref(desc), _ptr(u), _ptr(delta), _ptr(A), _ptr(Bm),
-                                    _ptr(Cm), _ptr(Dv), _ptr(y), _ptr(ckpt), _ptr(ws), nbytes,
-                                    ctypes.c_void_p(_stream_ptr(dev))))
-        _timer_stop(rec, ev0, "fwd", lambda: _record("fwd", u, Bm, in_dt, out_dt))
-    return y, ckpt
+    with torch.no_grad():
+        return _lib.native().scan_forward(u, delta, A, Bm, Cm, Dv, tok, _resolve_chunk(u.shape[1], chunk_len),
+                                          out_dtype, save_ckpt, False)
 
 
 def scan_backward(u, delta, A, Bm, Cm, Dv, dy, ckpt=None, tok=None, chunk_len=0, out_dtype=None):
     """Raw VJP launch.  Returns float32/out-dtype (du, ddelta, dA, dB, dC, dD)."""
-    u, delta, A, Bm, Cm, Dv, in_dt = _prepare(u, delta, A, Bm, Cm, Dv)
-    out_dt = out_dtype or in_dt
-    L = u.shape[1]
-    desc = _make_desc(u, Bm, in_dt, out_dt, tok, _resolve_chunk(L, chunk_len))
-    lib = _lib.lib()
-    dev = u.device
-    dy = dy.to(in_dt).contiguous()
-    if dy.shape != u.shape:
-        raise ValueError(f"dy shape {tuple(dy.shape)} != {tuple(u.shape)}")
-    with torch.cuda.device(dev):
-        du = torch.empty(u.shape, dtype=out_dt, device=dev)
-        ddelta = torch.empty(u.shape, dtype=torch.float32, device=dev)
-        dA = torch.empty(A.shape, dtype=torch.float32, device=dev)
-        dB = torch.empty_strided(Bm.shape, Bm.stride(), dtype=out_dt, device=dev)
-        dC = torch.empty_strided(Bm.shape, Bm.stride(), dtype=out_dt, device=dev)
-        dD = torch.empty(Dv.shape, dtype=torch.float32, device=dev)
-        which = 1 if ckpt is not None else 2
-        nbytes = _lib.check(lib.mvm_scan_workspace_bytes(ctypes.byref(desc), which))
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-        rec, ev0 = _timer_start()
-        _lib.check(lib.mvm_scan_bwd(ctypes.byref(desc), _ptr(u), _ptr(delta), _ptr(A), _ptr(Bm),
-                                    _ptr(Cm), _ptr(Dv), _ptr(ckpt), _ptr(dy), _ptr(du),
-                                    _ptr(ddelta), _ptr(dA), _ptr(dB), _ptr(dC), _ptr(dD),
-                                    _ptr(ws), nbytes, ctypes.c_void_p(_stream_ptr(dev))))
-        _timer_stop(rec, ev0, "bwd", lambda: _record("bwd", u, Bm, in_dt, out_dt))
-    return du, ddelta, dA, dB, dC, dD
+    with torch.no_grad():
+        return tuple(_lib.native().scan_backward(u, delta, A, Bm, Cm, Dv, dy, ckpt, tok,
+                                                 _resolve_chunk(u.shape[1], chunk_len), out_dtype))
 
 
 # ------------------------------------------------------------- fused form
-
-def _bkd(t):
-    """(b, t, k) strides of a (B, L, K, X) view."""
-    return t.stride(0), t.stride(1), t.stride(2)
-
-
-def _no_overlap(t):
-    """True when no two elements of t share memory: ordered by stride, each
-    dimension's stride clears the span of the smaller ones."""
-    span = 1
-    for st, sz in sorted((st, sz) for st, sz in zip(t.stride(), t.shape) if sz != 1):
-        if st < span:
-            return False
-        span = st * sz
-    return True
-
-
-def _fused_desc(u, delta_raw, Bm, y, z, tok, chunk_len, a_is_log=False):
-    fd = _lib.FusedDesc()
-    fd.a_is_log = int(bool(a_is_log))
-    fd.scan = _make_desc(u, Bm, torch.float32, torch.float32, tok, chunk_len)
-    fd.dt_stride_b, fd.dt_stride_t, fd.dt_stride_k = _bkd(delta_raw)
-    fd.y_stride_b, fd.y_stride_t, fd.y_stride_k = _bkd(y)
-    if z is not None:
-        fd.z_stride_b, fd.z_stride_t, fd.z_stride_k = _bkd(z)
-    return fd
-
-
-def _check_fused(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z):
-    bsz, L, K, D = u.shape
-    N = A.shape[-1]
-    if delta_raw.shape != u.shape or (z is not None and z.shape != u.shape):
-        raise ValueError("u, delta_raw and z must share the (B, L, K, D) shape")
-    if A.shape != (K, D, N) or Bm.shape != (bsz, L, K, N) or Cm.shape != Bm.shape:
-        raise ValueError("A must be (K, D, N) and B, C (B, L, K, N)")
-    if Dv.shape != (K, D) or (delta_bias is not None and delta_bias.shape != (K, D)):
-        raise ValueError("D and the dt bias must be (K, D)")
-    if Bm.stride() != Cm.stride():
-        raise ValueError("B and C must share strides")
-    ts = [u, delta_raw, A, Bm, Cm, Dv] + [t for t in (delta_bias, z) if t is not None]
-    _check_device(*ts)
-    for t in ts:
-        if t.dtype != torch.float32 or t.stride(-1) != 1:
-            raise ValueError("the fused scan takes float32 views with channel stride 1")
-    if not (A.is_contiguous() and Dv.is_contiguous()
-            and (delta_bias is None or delta_bias.is_contiguous())):
-        raise ValueError("A, D and the dt bias must be contiguous")
-
 
 def scan_fused_forward(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z, tok=None, chunk_len=0,
                        save=False, a_is_log=False):
@@ -293,29 +170,8 @@ def scan_fused_forward(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z, tok=None, chu
     (y, y_raw, ckpt): y (B, L, K, D) contiguous; y_raw and ckpt are saved for
     the backward when ``save`` (else None).
     """
-    _check_fused(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z)
-    dev = u.device
-    L = u.shape[1]
-    y = torch.empty(u.shape, dtype=torch.float32, device=dev)
-    fd = _fused_desc(u, delta_raw, Bm, y, z, tok, _resolve_chunk(L, chunk_len), a_is_log)
-    lib = _lib.lib()
-    with torch.cuda.device(dev):
-        y_raw = torch.empty_like(y) if (save and z is not None) else None
-        ckpt = None
-        if save:
-            ckpt = torch.empty(_lib.check(lib.mvm_scan_ckpt_elems(ctypes.byref(fd.scan))),
-                               dtype=torch.float32, device=dev)
-        nbytes = _lib.check(lib.mvm_scan_fused_workspace_bytes(ctypes.byref(fd), 0, int(z is not None)))
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-        rec, ev0 = _timer_start()
-        _lib.check(lib.mvm_scan_fused_fwd(
-            ctypes.byref(fd), _ptr(u), _ptr(delta_raw), _ptr(delta_bias), _ptr(A), _ptr(Bm),
-            _ptr(Cm), _ptr(Dv), _ptr(z), _ptr(y), _ptr(y_raw), _ptr(ckpt), _ptr(ws), nbytes,
-            ctypes.c_void_p(_stream_ptr(dev))))
-        _timer_stop(rec, ev0, "fwd", lambda: algorithmic_bytes_fused(
-            u.shape[0] * u.shape[2], L, u.shape[3], A.shape[-1], u.shape[2], z is not None,
-            delta_bias is not None)[0])
-    return y, y_raw, ckpt
+    return _lib.native().scan_fused_forward(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z, tok,
+                                            _resolve_chunk(u.shape[1], chunk_len), bool(save), bool(a_is_log))
 
 
 def scan_fused_backward(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z, y_raw, ckpt, dy, tok=None,
@@ -331,81 +187,9 @@ def scan_fused_backward(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z, y_raw, ckpt,
     dB, dC, dD, dz); ddelta_bias is None without a bias, dz None without a
     gate.
     """
-    _check_fused(u, delta_raw, delta_bias, A, Bm, Cm, Dv, z)
-    dev = u.device
-    L = u.shape[1]
-    if dy.shape != u.shape:
-        raise ValueError(f"dy shape {tuple(dy.shape)} != {tuple(u.shape)}")
-    # dy and y_raw share the y strides of the descriptor
-    ref = y_raw if (z is not None and y_raw is not None) else None
-    if ref is not None and not ref.is_contiguous():
-        raise ValueError("y_raw must be contiguous")
-    if dy.dtype != torch.float32 or not dy.is_contiguous():
-        dy = dy.float().contiguous()
-
-    def like(t):
-        # same strides as the primal (a layout with gaps allocates its span)
-        if not _no_overlap(t):
-            raise ValueError("a primal whose elements overlap (e.g. broadcast) needs an output view")
-        return torch.empty_strided(t.shape, t.stride(), dtype=torch.float32, device=dev)
-
-    du = like(u) if du is None else du
-    ddelta_raw = like(delta_raw) if ddelta_raw is None else ddelta_raw
-    if dB is None or dC is None:
-        dB, dC = like(Bm), like(Bm)
-    if dB.stride() != Bm.stride() or dC.stride() != Bm.stride():
-        raise ValueError("dB and dC must have the strides of B")
-    if z is not None and dz is None:
-        dz = like(z)
-    for t in (du, ddelta_raw, dB, dC) + ((dz,) if z is not None else ()):
-        if not _no_overlap(t):
-            raise ValueError("gradient views must not overlap themselves")
-    if (z is not None and dz.stride() != z.stride()) or ddelta_raw.stride() != delta_raw.stride() \
-            or du.stride() != u.stride():
-        raise ValueError("gradient views must have the strides of their primals")
-    ddelta_bias = torch.empty_like(delta_bias) if delta_bias is not None else None
-    dA = torch.empty(A.shape, dtype=torch.float32, device=dev)
-    dD = torch.empty(Dv.shape, dtype=torch.float32, device=dev)
-    fd = _fused_desc(u, delta_raw, Bm, dy, z, tok, _resolve_chunk(L, chunk_len), a_is_log)
-    lib = _lib.lib()
-    with torch.cuda.device(dev):
-        nbytes = _lib.check(lib.mvm_scan_fused_workspace_bytes(ctypes.byref(fd), 1, int(z is not None)))
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
-        rec, ev0 = _timer_start()
-        _lib.check(lib.mvm_scan_fused_bwd(
-            ctypes.byref(fd), _ptr(u), _ptr(delta_raw), _ptr(delta_bias), _ptr(A), _ptr(Bm),
-            _ptr(Cm), _ptr(Dv), _ptr(z), _ptr(y_raw), _ptr(ckpt), _ptr(dy), _ptr(du),
-            _ptr(ddelta_raw), _ptr(ddelta_bias), _ptr(dA), _ptr(dB), _ptr(dC), _ptr(dD), _ptr(dz),
-            _ptr(ws), nbytes, ctypes.c_void_p(_stream_ptr(dev))))
-        _timer_stop(rec, ev0, "bwd", lambda: algorithmic_bytes_fused(
-            u.shape[0] * u.shape[2], L, u.shape[3], A.shape[-1], u.shape[2], z is not None,
-            delta_bias is not None)[1])
-    return du, ddelta_raw, ddelta_bias, dA, dB, dC, dD, dz
-
-
-class _SelectiveScanFn(torch.autograd.Function):
-    """y = scan(u, delta, A, B, C, D) with the fused HIP VJP
-    (the custom_function + vjp pair of mamba_metal_fused.py:229-250)."""
-
-    @staticmethod
-    def forward(ctx, u, delta, A, Bm, Cm, Dv, tok, chunk_len, out_dtype, grad_mode):
-        # checkpoints only when a gradient can be asked for; grad mode is off
-        # inside forward, so the caller passes its own (grad_mode)
-        needs = grad_mode and any(ctx.needs_input_grad[:6])
-        y, ckpt = scan_forward(u, delta, A, Bm, Cm, Dv, tok, chunk_len, out_dtype, save_ckpt=needs)
-        ctx.chunk_len = chunk_len
-        ctx.out_dtype = out_dtype
-        ctx.in_dtypes = tuple(t.dtype for t in (u, delta, A, Bm, Cm, Dv))
-        if needs:
-            ctx.save_for_backward(u, delta, A, Bm, Cm, Dv, ckpt, tok)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        u, delta, A, Bm, Cm, Dv, ckpt, tok = ctx.saved_tensors
-        grads = scan_backward(u, delta, A, Bm, Cm, Dv, dy, ckpt, tok, ctx.chunk_len, ctx.out_dtype)
-        grads = tuple(g.to(dt) for g, dt in zip(grads, ctx.in_dtypes))
-        return grads + (None, None, None, None)
+    return _lib.native().scan_fused_backward(
+        u, delta_raw, delta_bias, A, Bm, Cm, Dv, z, y_raw, ckpt, dy, tok, _resolve_chunk(u.shape[1], chunk_len),
+        du, ddelta_raw, dB, dC, dz, bool(a_is_log))
 
 
 def check_permutation_table(table):
@@ -448,22 +232,14 @@ def selective_scan_directions(u, delta, A, B, C, D, seq_to_tok=None, chunk_len=0
         y, _ = scan_forward(u.detach(), delta.detach(), A.detach(), B.detach(), C.detach(),
                             D.detach(), seq_to_tok, _resolve_chunk(u.shape[1], chunk_len), out_dtype)
         return y
-    return _apply_scan(u, delta, A, B, C, D, seq_to_tok, chunk_len, out_dtype)
-
-
-def _apply_scan(u, delta, A, B, C, D, tok, chunk_len, out_dtype):
-    """_SelectiveScanFn.apply, saving checkpoints only when grad mode is on
-    (not under torch.no_grad / inference_mode)."""
-    return _SelectiveScanFn.apply(u, delta, A, B, C, D, tok, chunk_len, out_dtype,
-                                  torch.is_grad_enabled())
+    return _lib.native().scan(u, delta, A, B, C, D, seq_to_tok, _resolve_chunk(u.shape[1], chunk_len), out_dtype,
+                              False)
 
 
 def _scan3(x, delta, A, B, C, D, chunk_len, out_dtype=None):
     if x.dim() != 3:
         raise ValueError(f"x must be (B, L, D); got {tuple(x.shape)}")
-    y = _apply_scan(x.unsqueeze(2), delta.unsqueeze(2), A.unsqueeze(0), B.unsqueeze(2),
-                    C.unsqueeze(2), D.unsqueeze(0), None, chunk_len, out_dtype)
-    return y.squeeze(2)
+    return _lib.native().scan(x, delta, A, B, C, D, None, _resolve_chunk(x.shape[1], chunk_len), out_dtype, True)
 
 
 def selective_scan(x, delta, A, B, C, D, chunk_len=0, out_dtype=None):
@@ -498,9 +274,8 @@ def selective_scan_metal(x, delta, A, B, C, D):
     result is detached and no checkpoints are written)."""
     if x.dim() != 3:
         raise ValueError(f"x must be (B, L, D); got {tuple(x.shape)}")
-    y, _ = scan_forward(x.detach().unsqueeze(2), delta.detach().unsqueeze(2), A.detach().unsqueeze(0),
-                        B.detach().unsqueeze(2), C.detach().unsqueeze(2), D.detach().unsqueeze(0))
-    return y.squeeze(2)
+    with torch.no_grad():
+        return _lib.native().scan_forward(x, delta, A, B, C, D, None, 0, None, False, True)[0].detach()
 
 
 def selective_scan_metal_trainable(x, delta, A, B, C, D):
