@@ -41,7 +41,7 @@ typedef struct mvm_gemm_desc {
   int64_t batch;       /* 0..65535 / splits */
   int64_t lda, ldb, ldc;
   int64_t a_stride_batch, b_stride_batch, c_stride_batch;
-  int64_t b_seg;        /* 0, or a multiple of 32 that divides k */
+  int64_t b_seg;        /* 0, or a multiple of 16 that divides k */
   int64_t b_seg_stride;
   int32_t a_kmajor, b_kmajor;  /* 0 or 1 */
   int32_t accumulate;  /* 1: add to C */

@@ -778,8 +778,8 @@ int check_gemm(const mvm_gemm_desc* d) {
                         d->c_stride_batch, d->b_seg, d->b_seg_stride};
   for (int64_t v : st)
     if (v < 0) return fail(MVM_ERR_INVALID_ARG, "negative gemm stride");
-  if (d->b_seg > 0 && (d->b_seg % 32 != 0 || d->k % d->b_seg != 0))
-    return fail(MVM_ERR_INVALID_ARG, "gemm b_seg=%lld must be a multiple of 32 that divides k=%lld",
+  if (d->b_seg > 0 && (d->b_seg % 16 != 0 || d->k % d->b_seg != 0))
+    return fail(MVM_ERR_INVALID_ARG, "gemm b_seg=%lld must be a multiple of 16 that divides k=%lld",
                 (long long)d->b_seg, (long long)d->k);
   const int64_t bk = d->b_seg > 0 ? d->b_seg : d->k;
   if (d->lda < (d->a_kmajor ? d->k : d->m) || d->ldb < (d->b_kmajor ? bk : d->n))

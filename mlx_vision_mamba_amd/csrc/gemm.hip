@@ -444,6 +444,7 @@ void gemm_plan(GemmGeom& g) {
   float best = __builtin_inff();
   for (int c = 0; c < 2; ++c) {
     const TileCfg& t = kCfg[c];
+    if (g.seg < g.K && g.seg % t.bk != 0) continue;  // no step straddles two segments
     const float tiles = static_cast<float>(g.batch) * static_cast<float>((g.M + t.bm - 1) / t.bm) *
                         static_cast<float>((g.N + t.bn - 1) / t.bn);
     for (int ns = want > 0 ? want : 1; ns <= (want > 0 ? want : kMaxSplit); ++ns) {

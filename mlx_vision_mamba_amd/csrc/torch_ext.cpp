@@ -765,7 +765,7 @@ Tensor in_proj(const Tensor& h, const Tensor& W) {
 
 Tensor out_proj(const Tensor& y, const Tensor& W) {
   const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
-  if (usable(y, W, {E, D, K * D}) && (K == 1 || D % 32 == 0)) return OutProjFn::apply(y, W);
+  if (usable(y, W, {E, D, K * D}) && (K == 1 || D % 16 == 0)) return OutProjFn::apply(y, W);
   // one product over the concatenated directions (a reordered copy of W)
   auto shape = y.sizes().vec();
   shape.pop_back();

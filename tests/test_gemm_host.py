@@ -34,7 +34,7 @@ def _desc(**kw):
     (dict(m=-1), _lib.MVM_ERR_INVALID_ARG), (dict(lda=60), _lib.MVM_ERR_INVALID_ARG),
     (dict(lda=66), _lib.MVM_ERR_UNSUPPORTED), (dict(a_kmajor=0, lda=9), 0),
     (dict(a_kmajor=2), _lib.MVM_ERR_INVALID_ARG), (dict(splits=65), _lib.MVM_ERR_INVALID_ARG),
-    (dict(ldb=1 << 21), _lib.MVM_ERR_UNSUPPORTED), (dict(b_seg=16), _lib.MVM_ERR_INVALID_ARG),
+    (dict(ldb=1 << 21), _lib.MVM_ERR_UNSUPPORTED), (dict(b_seg=16, ldb=16), 0), (dict(b_seg=8), _lib.MVM_ERR_INVALID_ARG),
     (dict(b_seg=96), _lib.MVM_ERR_INVALID_ARG), (dict(batch=2), _lib.MVM_ERR_INVALID_ARG),
     (dict(ldc=7), _lib.MVM_ERR_INVALID_ARG), (dict(m=1 << 31), _lib.MVM_ERR_UNSUPPORTED),
 ])

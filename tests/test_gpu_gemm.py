@@ -85,7 +85,7 @@ def test_error_no_larger_than_float32(cuda, m, n, k, shift):
     assert err(C) <= err(F.linear(A, B)), (err(C), err(F.linear(A, B)))
 
 
-@pytest.mark.parametrize("K,D", [(3, 32), (4, 96), (2, 160)])
+@pytest.mark.parametrize("K,D", [(3, 32), (4, 96), (2, 160), (2, 16), (2, 400), (3, 48)])
 def test_segments(cuda, K, D):
     """One product over K weight matrices that lie apart."""
     gen = torch.Generator().manual_seed(K)
@@ -135,7 +135,7 @@ def test_special_values_as_float32(cuda, akm, bkm, k, splits):
 @pytest.mark.parametrize("B,n,K,D,E", [(2, 37, 1, 24, 12), (3, 50, 4, 64, 40), (0, 5, 2, 32, 16), (1, 9, 2, 40, 20)])
 def test_projections_match_autograd(cuda, B, n, K, D, E):
     """in_proj / out_proj (also where the kernels do not take the shape:
-    Din = 40 in two directions) against float64 autograd."""
+    Din = 40 in two directions, not a multiple of 16) against float64 autograd."""
     gen = torch.Generator().manual_seed(1)
     h = torch.randn(B, n, E, generator=gen).cuda().requires_grad_()
     Wi = torch.randn(K * 2 * D, E, generator=gen).cuda().requires_grad_()
