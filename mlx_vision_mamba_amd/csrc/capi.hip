@@ -52,19 +52,24 @@ constexpr int64_t kMaxSeqlen = INT32_MAX - 64;
 // Time-chunk length.  One chunk (no carry passes) when the (batch x
 // direction x channel-block) grid alone gives >= 4096 waves (four per SIMD
 // on the 256-CU MI355X); otherwise the sequence is cut until the main passes
-// launch ~16k waves, into at most ceil(tiles / 2) chunks (2 tiles = 32
-// positions each; the last may hold one).  Measured on MI355X: B=32 L=196
-// D=3072 is fastest unchunked; B=8 L=16384 D=1536 at 512-768 positions per
-// chunk; B=2 L=196 D=1536 at 32 (fwd + VJP graph replay 50.3 us, against
-// 54.8 at 48 and 60.7 at 16).
+// launch ~16k waves, but into chunks of at least 4 tiles (64 positions) while
+// those give 2048 waves, of 3 tiles while those give 1536, and of 2 below: a
+// shorter chunk repeats more of the per-chunk work (prologue, aggregates,
+// carry) than its waves return.  Measured on MI355X, forward + VJP us by
+// positions per chunk: B=3 L=1037 D=1000: 32 111, 64 103, 96 113; B=16 L=512
+// D=768: 32 174, 48 168, 64 156 (8 chunks: folded without a carry pass);
+// B=1 L=4096 D=768: 32 128, 64 109; B=30 L=300 D=300: 32 106, 64 93; B=10
+// L=331 D=400: 32 68, 48 60 (7 chunks), 64 69; B=2 L=196 D=1536: 32 44, 48 46,
+// 64 54; B=32 L=196 D=3072 is fastest unchunked; B=8 L=16384 D=1536 flat over
+// 256-1024.
 int64_t pick_chunk_len(const mvm_scan_desc* d) {
   if (d->chunk_len > 0) return d->chunk_len;
   const int64_t tiles = ceil_div(d->seqlen, mvm::kSub);
   const int64_t waves = d->batch * d->ndir * ceil_div(d->dim, mvm::kChPerBlock) * 4;
   int64_t nchunk = 1;
   if (waves < 4096) nchunk = ceil_div(16384, std::max<int64_t>(waves, 1));
-  nchunk = std::min(nchunk, std::max<int64_t>(1, (tiles + 1) / 2));
-  const int64_t tiles_per_chunk = ceil_div(tiles, nchunk);
+  const int64_t least = waves * ceil_div(tiles, 4) >= 2048 ? 4 : (waves * ceil_div(tiles, 3) >= 1536 ? 3 : 2);
+  const int64_t tiles_per_chunk = nchunk == 1 ? tiles : std::max(least, ceil_div(tiles, nchunk));
   return std::max<int64_t>(1, tiles_per_chunk) * mvm::kSub;
 }
 

@@ -177,16 +177,26 @@ scan_bwd_carry_kernel(Geom gm, BwdBufs bf) {
   const int64_t bk = idx / (kStatePad * gm.D);
   const int64_t k = bk % gm.K;
   const float a2 = n < gm.N ? load_A(bf.A, (k * gm.D + d) * gm.N + n, gm.a_log) * kLog2e : 0.f;
+  // loaded batch by batch, as in scan_fwd_carry_kernel
+  const int64_t step = gm.D * kStatePad;
+  float* pm = bf.agg_mu + (bk * gm.nchunk * gm.D + d) * kStatePad + n;
+  const float* ps = bf.agg_s + bk * gm.nchunk * gm.D + d;
   float carry = 0.f;
-  for (int64_t c = gm.nchunk - 1; c >= 0; --c) {
-    const int64_t slot = (bk * gm.nchunk + c) * gm.D + d;
-    float a = 0.f, s = 0.f;
-    if (c >= 1) {
-      a = bf.agg_mu[slot * kStatePad + n];
-      s = bf.agg_s[slot];
+  for (int64_t c0 = gm.nchunk - 1; c0 >= 0; c0 -= kCarryBatch) {
+    float a[kCarryBatch], s[kCarryBatch];
+#pragma unroll
+    for (int i = 0; i < kCarryBatch; ++i) {
+      const int64_t c = c0 - i >= 1 ? c0 - i : gm.nchunk - 1;  // (the first chunk has no aggregate)
+      a[i] = pm[c * step];
+      s[i] = ps[c * gm.D];
     }
-    bf.agg_mu[slot * kStatePad + n] = carry;
-    carry = fmaf(fast_exp2(a2 * s), carry, a);
+#pragma unroll
+    for (int i = 0; i < kCarryBatch; ++i) {
+      if (c0 - i >= 0) {
+        pm[(c0 - i) * step] = carry;
+        carry = fmaf(fast_exp2(a2 * s[i]), carry, a[i]);
+      }
+    }
   }
 }
 

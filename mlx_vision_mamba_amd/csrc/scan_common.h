@@ -28,6 +28,8 @@ constexpr float kLn2 = 0.6931471805599453f;
 // aggregates it needs itself (one launch fewer); beyond it a separate carry
 // pass folds them once, so no block waits on a long chain of loads.
 constexpr int64_t kFoldMax = 8;
+// chunks whose aggregates a carry pass has in flight together
+constexpr int kCarryBatch = 8;
 
 struct bf16_t {
   uint16_t bits;

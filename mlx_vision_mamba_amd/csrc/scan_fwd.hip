@@ -280,16 +280,28 @@ scan_fwd_carry_kernel(Geom gm, FwdBufs bf) {
   const int64_t bk = idx / (kStatePad * gm.D);
   const int64_t k = bk % gm.K;
   const float a2 = n < gm.N ? load_A(bf.A, (k * gm.D + d) * gm.N + n, gm.a_log) * kLog2e : 0.f;
+  // the aggregates of a batch of chunks are loaded together (from in-bounds
+  // slots) before the first is folded: one memory latency per batch instead
+  // of one per chunk
+  const int64_t step = gm.D * kStatePad;
+  float* ph = bf.agg_h + (bk * gm.nchunk * gm.D + d) * kStatePad + n;
+  const float* ps = bf.agg_s + bk * gm.nchunk * gm.D + d;
   float carry = 0.f;
-  for (int64_t c = 0; c < gm.nchunk; ++c) {
-    const int64_t slot = (bk * gm.nchunk + c) * gm.D + d;
-    float e = 0.f, s = 0.f;
-    if (c + 1 < gm.nchunk) {
-      e = bf.agg_h[slot * kStatePad + n];
-      s = bf.agg_s[slot];
+  for (int64_t c0 = 0; c0 < gm.nchunk; c0 += kCarryBatch) {
+    float e[kCarryBatch], s[kCarryBatch];
+#pragma unroll
+    for (int i = 0; i < kCarryBatch; ++i) {
+      const int64_t c = c0 + i + 1 < gm.nchunk ? c0 + i : 0;  // (the last chunk has no aggregate)
+      e[i] = ph[c * step];
+      s[i] = ps[c * gm.D];
     }
-    bf.agg_h[slot * kStatePad + n] = carry;
-    carry = fmaf(fast_exp2(a2 * s), carry, e);
+#pragma unroll
+    for (int i = 0; i < kCarryBatch; ++i) {
+      if (c0 + i < gm.nchunk) {
+        ph[(c0 + i) * step] = carry;
+        carry = fmaf(fast_exp2(a2 * s[i]), carry, e[i]);
+      }
+    }
   }
 }
 
