@@ -7,14 +7,16 @@
  * and their gradients, for all directions of a block at once (:562-566).
  * For each batch index q:
  *
- *   C_q[i, j] (+)= sum_p A_q[i, p] * B_q[p, j]      i < m, j < n, p < k
+ *   C_q[i, j] = sum_p A_q[i, p] * B_q[p, j] (+ add_q[i, j])    i < m, j < n, p < k
  *
  * Operands are float32; each lies in one of two layouts:
  *   a_kmajor = 1: A_q[i, p] at A[q * a_stride_batch + i * lda + p]
  *   a_kmajor = 0: A_q[i, p] at A[q * a_stride_batch + p * lda + i]
  *   b_kmajor = 1: B_q[p, j] at B[q * b_stride_batch + j * ldb + p]
  *   b_kmajor = 0: B_q[p, j] at B[q * b_stride_batch + p * ldb + j]
- * C_q[i, j] is C[q * c_stride_batch + i * ldc + j].  With b_seg > 0 the sum
+ * C_q[i, j] is C[q * c_stride_batch + i * ldc + j], add_q the same of add:
+ * NULL, C itself (the products are added to it), or another buffer of C's
+ * layout that does not overlap it (a block's residual).  With b_seg > 0 the sum
  * over p runs over segments of b_seg values whose B parts lie b_seg_stride
  * elements apart: p counts as p % b_seg in the addresses above, plus
  * (p / b_seg) * b_seg_stride (the out_proj weights of K directions, each a
@@ -44,7 +46,7 @@ typedef struct mvm_gemm_desc {
   int64_t b_seg;        /* 0, or a multiple of 16 that divides k */
   int64_t b_seg_stride;
   int32_t a_kmajor, b_kmajor;  /* 0 or 1 */
-  int32_t accumulate;  /* 1: add to C */
+  int32_t reserved;    /* must be 0 */
   int32_t splits;      /* parts the sum over p is cut into; 0: chosen by the library */
 } mvm_gemm_desc;
 
@@ -57,9 +59,9 @@ int mvm_gemm_validate(const mvm_gemm_desc* desc);
 int64_t mvm_gemm_workspace_bytes(const mvm_gemm_desc* desc);
 
 /* From k = 32 up k-major operands must be 16-byte aligned; the workspace must
- * be 256-byte aligned.  k = 0 writes zeros (accumulate: leaves C). */
-int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, float* C,
-                 void* workspace, size_t workspace_bytes, void* stream);
+ * be 256-byte aligned.  With k = 0 the products are zero. */
+int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, const float* add,
+                 float* C, void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -85,7 +85,7 @@ class GemmDesc(ctypes.Structure):
         ("lda", _i64), ("ldb", _i64), ("ldc", _i64),
         ("a_stride_batch", _i64), ("b_stride_batch", _i64), ("c_stride_batch", _i64),
         ("b_seg", _i64), ("b_seg_stride", _i64),
-        ("a_kmajor", _i32), ("b_kmajor", _i32), ("accumulate", _i32), ("splits", _i32),
+        ("a_kmajor", _i32), ("b_kmajor", _i32), ("reserved", _i32), ("splits", _i32),
     ]
 
 
@@ -139,7 +139,7 @@ SIGNATURES = {
 GEMM_SIGNATURES = {
     "mvm_gemm_validate": (ctypes.c_int, [ctypes.POINTER(GemmDesc)]),
     "mvm_gemm_workspace_bytes": (_i64, [ctypes.POINTER(GemmDesc)]),
-    "mvm_gemm_f32": (ctypes.c_int, [ctypes.POINTER(GemmDesc)] + [_vp] * 4 + [ctypes.c_size_t, _vp]),
+    "mvm_gemm_f32": (ctypes.c_int, [ctypes.POINTER(GemmDesc)] + [_vp] * 5 + [ctypes.c_size_t, _vp]),
 }
 
 _lib = None

@@ -775,8 +775,9 @@ int check_gemm(const mvm_gemm_desc* d) {
   if (d->m > kGemmMaxDim || d->n > kGemmMaxDim || d->k > kGemmMaxDim || d->batch > 65535)
     return fail(MVM_ERR_UNSUPPORTED, "gemm size too large (m=%lld n=%lld k=%lld batch=%lld)",
                 (long long)d->m, (long long)d->n, (long long)d->k, (long long)d->batch);
-  if ((d->a_kmajor | d->b_kmajor | d->accumulate) & ~1)
+  if ((d->a_kmajor | d->b_kmajor) & ~1)
     return fail(MVM_ERR_INVALID_ARG, "gemm flags must be 0 or 1");
+  if (d->reserved != 0) return fail(MVM_ERR_INVALID_ARG, "gemm desc reserved field must be 0");
   if (d->splits < 0 || d->splits > 64)
     return fail(MVM_ERR_INVALID_ARG, "gemm splits=%d must be 0..64", d->splits);
   const int64_t st[] = {d->lda, d->ldb, d->ldc, d->a_stride_batch, d->b_stride_batch,
@@ -810,7 +811,6 @@ int gemm_geom(const mvm_gemm_desc* d, mvm::GemmGeom& g) {
   g.seg = static_cast<int32_t>(d->b_seg > 0 ? d->b_seg : std::max<int64_t>(d->k, 1));
   g.seg_stride = d->b_seg > 0 ? d->b_seg_stride : 0;
   g.a_km = d->a_kmajor; g.b_km = d->b_kmajor;
-  g.accumulate = d->accumulate;
   g.nsplit = d->splits;
   mvm::gemm_plan(g);
   if (d->batch * g.nsplit > 65535 || ceil_div(d->m, 64) * ceil_div(d->n, 64) > INT32_MAX / 256)
@@ -838,13 +838,13 @@ int64_t mvm_gemm_workspace_bytes(const mvm_gemm_desc* desc) {
   return static_cast<int64_t>(align_up(sizeof(float) * mvm::gemm_partial_floats(g)));
 }
 
-int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, float* C,
-                 void* workspace, size_t workspace_bytes, void* stream) {
+int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, const float* add,
+                 float* C, void* workspace, size_t workspace_bytes, void* stream) {
   int rc = check_gemm(desc);
   mvm::GemmGeom g;
   if (rc == MVM_OK) rc = gemm_geom(desc, g);
   if (rc != MVM_OK) return rc;
-  if (g.M == 0 || g.N == 0 || g.batch == 0 || (g.K == 0 && g.accumulate)) return ok();
+  if (g.M == 0 || g.N == 0 || g.batch == 0) return ok();
   if (!C || (g.K > 0 && (!A || !B))) return fail(MVM_ERR_INVALID_ARG, "mvm_gemm_f32: NULL pointer");
   if (g.K >= 32 &&
       ((g.a_km && (reinterpret_cast<uintptr_t>(A) & 15u)) || (g.b_km && (reinterpret_cast<uintptr_t>(B) & 15u))))
@@ -854,7 +854,7 @@ int mvm_gemm_f32(const mvm_gemm_desc* desc, const float* A, const float* B, floa
     rc = check_ws("mvm_gemm_f32", workspace, workspace_bytes, need);
     if (rc != MVM_OK) return rc;
   }
-  return hip_status(mvm::launch_gemm(g, A, B, C, static_cast<float*>(workspace),
+  return hip_status(mvm::launch_gemm(g, A, B, add, C, static_cast<float*>(workspace),
                                      static_cast<hipStream_t>(stream)),
                     "mvm_gemm_f32 launch");
 }

@@ -159,7 +159,7 @@ struct Operand {
 template <int BM, int BN, int BK, int OCC, bool AKM, bool BKM>
 __global__ void __launch_bounds__(kThreads, OCC)
 gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B,
-            float* __restrict__ C) {
+            const float* add_src, float* C) {
   constexpr int MT = BM / 64, NT = BN / 64;  // 32 x 32 tiles of a wave
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][3][BM][BK];
   __shared__ __attribute__((aligned(16))) uint16_t sB[2][3][BN][BK];
@@ -335,9 +335,10 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
 
   // split: partial products side by side, (q, part, m, n)
   const bool split = g.nsplit > 1;
-  float* __restrict__ Cq = split ? C + static_cast<int64_t>(blockIdx.z) * g.M * g.N : C + q * g.sc;
+  float* Cq = split ? C + static_cast<int64_t>(blockIdx.z) * g.M * g.N : C + q * g.sc;
   const int64_t ldc = split ? g.N : g.ldc;
-  const bool add = !split && g.accumulate;
+  const bool add = !split && add_src != nullptr;  // (may be C itself)
+  const float* Sq = add_src + (add ? q * g.sc : 0);
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -351,7 +352,7 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
         float old[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          old[r] = Cq[min(row0 + 8 * (r / 4) + (r & 3), g.M - 1) * ldc + min(col, g.N - 1)];
+          old[r] = Sq[min(row0 + 8 * (r / 4) + (r & 3), g.M - 1) * ldc + min(col, g.N - 1)];
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] += old[r];
       }
@@ -363,10 +364,10 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
     }
 }
 
-// C (+)= the sum of the partial products, left to right
+// C = the sum of the partial products, left to right (+ add_src)
 template <typename V>
 __global__ void __launch_bounds__(kThreads)
-gemm_reduce_kernel(GemmGeom g, const float* __restrict__ part, float* __restrict__ C) {
+gemm_reduce_kernel(GemmGeom g, const float* __restrict__ part, const float* add_src, float* C) {
   constexpr int W = sizeof(V) / sizeof(float);
   const int64_t mn = static_cast<int64_t>(g.M) * g.N;
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * W;
@@ -374,7 +375,7 @@ gemm_reduce_kernel(GemmGeom g, const float* __restrict__ part, float* __restrict
   const int64_t q = blockIdx.y;
   const float* p = part + q * g.nsplit * mn + i;
   const int64_t row = i / g.N;
-  float* c = C + q * g.sc + row * g.ldc + (i - row * g.N);
+  const int64_t at = q * g.sc + row * g.ldc + (i - row * g.N);
   float s[W];
   V v = *reinterpret_cast<const V*>(p);
 #pragma unroll
@@ -384,14 +385,14 @@ gemm_reduce_kernel(GemmGeom g, const float* __restrict__ part, float* __restrict
 #pragma unroll
     for (int e = 0; e < W; ++e) s[e] += reinterpret_cast<const float*>(&v)[e];
   }
-  if (g.accumulate) {
-    v = *reinterpret_cast<const V*>(c);
+  if (add_src != nullptr) {
+    v = *reinterpret_cast<const V*>(add_src + at);
 #pragma unroll
     for (int e = 0; e < W; ++e) s[e] += reinterpret_cast<const float*>(&v)[e];
   }
 #pragma unroll
   for (int e = 0; e < W; ++e) reinterpret_cast<float*>(&v)[e] = s[e];
-  *reinterpret_cast<V*>(c) = v;
+  *reinterpret_cast<V*>(C + at) = v;
 }
 
 // Tile shapes: 2 workgroups on a CU (by VGPRs), 3 (by LDS).
@@ -408,18 +409,18 @@ constexpr float kBytesPerUs = 4.5e6f;  // HBM, streaming
 constexpr int kMaxSplit = 24;
 
 template <int CFG, bool AKM, bool BKM>
-void launch_cfg(const GemmGeom& g, const float* A, const float* B, float* C, hipStream_t s) {
+void launch_cfg(const GemmGeom& g, const float* A, const float* B, const float* add, float* C, hipStream_t s) {
   constexpr TileCfg c = kCfg[CFG];
   const unsigned nt = static_cast<unsigned>((g.M + c.bm - 1) / c.bm) * static_cast<unsigned>((g.N + c.bn - 1) / c.bn);
   hipLaunchKernelGGL((gemm_kernel<c.bm, c.bn, c.bk, c.occ, AKM, BKM>),
-                     dim3(nt, 1, static_cast<unsigned>(g.batch * g.nsplit)), dim3(kThreads), 0, s, g, A, B, C);
+                     dim3(nt, 1, static_cast<unsigned>(g.batch * g.nsplit)), dim3(kThreads), 0, s, g, A, B, add, C);
 }
 template <int CFG>
-void launch_layout(const GemmGeom& g, const float* A, const float* B, float* C, hipStream_t s) {
+void launch_layout(const GemmGeom& g, const float* A, const float* B, const float* add, float* C, hipStream_t s) {
   if (g.a_km)
-    g.b_km ? launch_cfg<CFG, true, true>(g, A, B, C, s) : launch_cfg<CFG, true, false>(g, A, B, C, s);
+    g.b_km ? launch_cfg<CFG, true, true>(g, A, B, add, C, s) : launch_cfg<CFG, true, false>(g, A, B, add, C, s);
   else
-    g.b_km ? launch_cfg<CFG, false, true>(g, A, B, C, s) : launch_cfg<CFG, false, false>(g, A, B, C, s);
+    g.b_km ? launch_cfg<CFG, false, true>(g, A, B, add, C, s) : launch_cfg<CFG, false, false>(g, A, B, add, C, s);
 }
 
 }  // namespace
@@ -427,11 +428,11 @@ void launch_layout(const GemmGeom& g, const float* A, const float* B, float* C, 
 // The tile shape and split with the least estimated time: the steps of the
 // busiest CU, writing C, and with a split the partial products (written and
 // read) and the second launch.  Measured (estimated) us on MI355X, the BLAS
-// library's time last: 6272 x 6144 x 384: 128-tiles unsplit 207 (189), 64-tiles
-// 241, library 248-290; 6272 x 384 x 6144: 128-tiles in 3 parts 187 (194),
-// unsplit 310, 8 parts 197, library 262; 196 x 1536 x 384: 64-tiles unsplit
-// 10.0 (6.3 + launch), 128-tiles 22.8, library 19.6; 196 x 384 x 768: 64-tiles
-// in 4-8 parts 10.3, unsplit 15.9, library 19.2.
+// library's time last: 6272 x 6144 x 384: 128-tiles unsplit 207 (197), 64-tiles
+// 241, library 248-290; 6272 x 384 x 6144: 128-tiles in 3 parts 187 (191), in 4
+// (76 workgroups past a full round) 222 (233), unsplit 310, library 262; 196 x
+// 1536 x 384: 64-tiles unsplit 10.0 (6.3 + launch), 128-tiles 22.8, library
+// 19.6; 196 x 384 x 768: 64-tiles in 4-8 parts 10.3, unsplit 15.9, library 19.2.
 void gemm_plan(GemmGeom& g) {
   const int want = g.nsplit;  // > 0: the caller's split
   if (g.K < 32) {  // less than a step of the small tile, which loads it value by value
@@ -440,23 +441,27 @@ void gemm_plan(GemmGeom& g) {
     g.kper = 32;
     return;
   }
-  const float mn4 = 4.f * static_cast<float>(g.batch) * static_cast<float>(g.M) * static_cast<float>(g.N);
+  const int64_t mn4 = int64_t{4} * g.batch * g.M * g.N;
+  const float write = static_cast<float>(mn4) / kBytesPerUs;
   float best = __builtin_inff();
   for (int c = 0; c < 2; ++c) {
     const TileCfg& t = kCfg[c];
     if (g.seg < g.K && g.seg % t.bk != 0) continue;  // no step straddles two segments
-    const float tiles = static_cast<float>(g.batch) * static_cast<float>((g.M + t.bm - 1) / t.bm) *
-                        static_cast<float>((g.N + t.bn - 1) / t.bn);
+    const int64_t tiles = int64_t{g.batch} * ((g.M + t.bm - 1) / t.bm) * ((g.N + t.bn - 1) / t.bn);
+    const int64_t slots = int64_t{kCUs} * t.occ;
     for (int ns = want > 0 ? want : 1; ns <= (want > 0 ? want : kMaxSplit); ++ns) {
-      // (at least 64 values of k per part; partial products of at most 1 GiB)
+      // (at least 64 values of k per part, partial products of at most 1 GiB,
+      // and no further split of what fills the chip four times)
       if (want == 0 && ns > 1 &&
-          (g.K / ns < 64 || mn4 * ns > 1073741824.f || static_cast<int64_t>(g.batch) * ns > 65535)) break;
-      const int kper = static_cast<int>((static_cast<int64_t>(g.K) + ns - 1) / ns + t.bk - 1) / t.bk * t.bk;
-      const float steps = static_cast<float>(kper / t.bk);
-      const float n = tiles * static_cast<float>(ns);
-      const float load = n <= kCUs * t.occ ? __builtin_ceilf(n / kCUs) : n / kCUs + 0.3f;
-      float us = steps * (load <= 1.f ? t.alone : t.shared * load) + mn4 / kBytesPerUs;
-      if (ns > 1) us += 3.f + 2.f * static_cast<float>(ns) * mn4 / kBytesPerUs;
+          (g.K < 64 * ns || mn4 * ns > (int64_t{1} << 30) || int64_t{g.batch} * ns > 65535 ||
+           tiles * (ns - 1) > 4 * slots)) break;
+      const int kper = static_cast<int>((int64_t{g.K} + ns - 1) / ns + t.bk - 1) / t.bk * t.bk;
+      // whole rounds of t.occ workgroups per CU, then the rest
+      const int64_t n = tiles * ns, rounds = n / slots, rest = (n % slots + kCUs - 1) / kCUs;
+      float us = static_cast<float>(kper / t.bk) *
+                     (t.shared * static_cast<float>(rounds * t.occ + (rest == 1 ? 0 : rest)) +
+                      (rest == 1 ? t.alone : 0.f)) + write;
+      if (ns > 1) us += 3.f + 3.f * static_cast<float>(ns) * write;
       if (us < best) {
         best = us;
         g.cfg = c;
@@ -471,22 +476,22 @@ int64_t gemm_partial_floats(const GemmGeom& g) {
   return g.nsplit > 1 ? static_cast<int64_t>(g.batch) * g.nsplit * g.M * g.N : 0;
 }
 
-hipError_t launch_gemm(const GemmGeom& g, const float* A, const float* B, float* C, float* part,
-                       hipStream_t s) {
+hipError_t launch_gemm(const GemmGeom& g, const float* A, const float* B, const float* add, float* C,
+                       float* part, hipStream_t s) {
   float* out = g.nsplit > 1 ? part : C;
   switch (g.cfg) {
-    case 0: launch_layout<0>(g, A, B, out, s); break;
-    default: launch_layout<1>(g, A, B, out, s); break;
+    case 0: launch_layout<0>(g, A, B, add, out, s); break;
+    default: launch_layout<1>(g, A, B, add, out, s); break;
   }
   if (g.nsplit > 1) {
     const bool vec = g.N % 4 == 0 && g.ldc % 4 == 0 && g.sc % 4 == 0 &&
-                     (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
+                     ((reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(add)) & 15u) == 0;
     const int64_t n = static_cast<int64_t>(g.M) * g.N / (vec ? 4 : 1);
     const dim3 grid(static_cast<unsigned>((n + kThreads - 1) / kThreads), static_cast<unsigned>(g.batch));
     if (vec)
-      hipLaunchKernelGGL((gemm_reduce_kernel<float4>), grid, dim3(kThreads), 0, s, g, part, C);
+      hipLaunchKernelGGL((gemm_reduce_kernel<float4>), grid, dim3(kThreads), 0, s, g, part, add, C);
     else
-      hipLaunchKernelGGL((gemm_reduce_kernel<float>), grid, dim3(kThreads), 0, s, g, part, C);
+      hipLaunchKernelGGL((gemm_reduce_kernel<float>), grid, dim3(kThreads), 0, s, g, part, add, C);
   }
   return hipGetLastError();
 }

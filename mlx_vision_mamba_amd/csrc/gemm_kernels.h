@@ -16,7 +16,6 @@ struct GemmGeom {
   int32_t seg;           // B segment length along k (K when there is one)
   int64_t seg_stride;
   int32_t a_km, b_km;    // 1: k is the contiguous index
-  int32_t accumulate;
   int32_t cfg;           // tile shape (gemm.hip)
   int32_t nsplit, kper;  // the sum over k in nsplit parts of kper
 };
@@ -26,7 +25,8 @@ struct GemmGeom {
 void gemm_plan(GemmGeom& g);
 // float32 elements of the partial-product buffer (0 without a split)
 int64_t gemm_partial_floats(const GemmGeom& g);
-hipError_t launch_gemm(const GemmGeom& g, const float* A, const float* B, float* C, float* part,
-                       hipStream_t s);
+// add: nullptr, or what is added to the products, laid out as C (may be C)
+hipError_t launch_gemm(const GemmGeom& g, const float* A, const float* B, const float* add, float* C,
+                       float* part, hipStream_t s);
 
 }  // namespace mvm

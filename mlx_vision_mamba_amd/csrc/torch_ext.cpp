@@ -607,12 +607,13 @@ std::vector<Tensor> norm(const Tensor& x, const Tensor& w, const Tensor& b, doub
 
 // ---------------------------------------------------------------- products
 
-void gemm(const Tensor& A, const Tensor& B, const Tensor& C, mvm_gemm_desc d) {
+// C = A @ B (+ add, laid out as C)
+void gemm(const Tensor& A, const Tensor& B, const Tensor& C, mvm_gemm_desc d, const Tensor& add = Tensor()) {
   c10::OptionalDeviceGuard guard(C.device());
   const int64_t nbytes = check(mvm_gemm_workspace_bytes(&d));
   Tensor ws;
   if (nbytes > 0) ws = workspace(nbytes, C);
-  check(mvm_gemm_f32(&d, fp(A), fp(B), fpm(C), ws.defined() ? ws.mutable_data_ptr() : nullptr,
+  check(mvm_gemm_f32(&d, fp(A), fp(B), fp(add), fpm(C), ws.defined() ? ws.mutable_data_ptr() : nullptr,
                      static_cast<size_t>(nbytes), stream_of(C)));
 }
 
@@ -648,8 +649,7 @@ void batched(const Tensor& A, const Tensor& B, Tensor& out, bool ta, bool tb, bo
     auto d = gemm_desc(m, n, k, A.stride(1), B.stride(1), out.stride(1), !ta, tb);
     d.batch = q;
     d.a_stride_batch = A.stride(0); d.b_stride_batch = B.stride(0); d.c_stride_batch = out.stride(0);
-    d.accumulate = accumulate;
-    gemm(A, B, out, d);
+    gemm(A, B, out, d, accumulate ? out : Tensor());
     return;
   }
   const Tensor Av = ta ? A.transpose(1, 2) : A, Bv = tb ? B.transpose(1, 2) : B;
@@ -711,9 +711,10 @@ struct InProjFn : Function<InProjFn> {
 
 // sum over k of y (..., K, D)[k] @ W (K, E, D)[k]^T: the K weight matrices
 // are read where they lie, as one product over K * D, and their gradient
-// comes out in the same layout, so no reordered copy of either is made
+// comes out in the same layout, so no reordered copy of either is made.  A
+// residual is added in the product's epilogue
 struct OutProjFn : Function<OutProjFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& y, const Tensor& W) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& y, const Tensor& W, const OptTensor& res) {
     const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
     const Tensor y2 = dense(y.reshape({-1, K * D}));
     const int64_t M = y2.size(0);
@@ -723,8 +724,9 @@ struct OutProjFn : Function<OutProjFn> {
       d.b_seg = D;
       d.b_seg_stride = E * D;
     }
-    gemm(y2, W, out, d);
+    gemm(y2, W, out, d, res.has_value() ? res->reshape({M, E}).contiguous() : Tensor());
     ctx->save_for_backward({y2, W});
+    ctx->saved_data["res"] = res.has_value();
     ctx->saved_data["shape"] = y.sizes().vec();
     auto shape = y.sizes().vec();
     shape.pop_back();
@@ -754,7 +756,7 @@ struct OutProjFn : Function<OutProjFn> {
       d.c_stride_batch = E * D;
       gemm(g2, y2, dW, d);
     }
-    return {dy, dW};
+    return {dy, dW, ctx->saved_data["res"].toBool() ? g[0] : Tensor()};
   }
 };
 
@@ -763,14 +765,23 @@ Tensor in_proj(const Tensor& h, const Tensor& W) {
   return at::linear(h, W);
 }
 
-Tensor out_proj(const Tensor& y, const Tensor& W) {
+Tensor out_proj(const Tensor& y, const Tensor& W, const OptTensor& res) {
   const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
-  if (usable(y, W, {E, D, K * D}) && (K == 1 || D % 16 == 0)) return OutProjFn::apply(y, W);
+  if (usable(y, W, {E, D, K * D}) && (K == 1 || D % 16 == 0)) {
+    auto shape = y.sizes().vec();
+    shape.pop_back();
+    shape.back() = E;
+    if (!res.has_value()) return OutProjFn::apply(y, W, res);
+    if (res->scalar_type() == at::kFloat && res->device() == y.device() && res->sizes() == shape)
+      return OutProjFn::apply(y, W, res);
+    return *res + OutProjFn::apply(y, W, OptTensor());
+  }
   // one product over the concatenated directions (a reordered copy of W)
   auto shape = y.sizes().vec();
   shape.pop_back();
   shape.back() = K * D;
-  return at::linear(y.reshape(shape), W.permute({1, 0, 2}).reshape({E, K * D}));
+  const Tensor out = at::linear(y.reshape(shape), W.permute({1, 0, 2}).reshape({E, K * D}));
+  return res.has_value() ? *res + out : out;
 }
 
 // -------------------------------------------------------------- block core
@@ -912,11 +923,11 @@ struct CoreFn : Function<CoreFn> {
 };
 
 // K MambaBlocks on one (B, N, E) input, block k scanning in the order of
-// tok[k]; the sum of their outputs.  params: the nine kinds of
+// tok[k]; the sum of their outputs, and of the residual when there is one.  params: the nine kinds of
 // mamba_block.STACKED_PARAMS, kind-major, K each; stacks: the buffers whose
 // leading K slices they are (empty: a single block).
 Tensor directional(const Tensor& h, const std::vector<Tensor>& params, const std::vector<Tensor>& stacks,
-                   int64_t K, const OptTensor& tok_, int64_t chunk_len, bool detach) {
+                   int64_t K, const OptTensor& tok_, int64_t chunk_len, bool detach, const OptTensor& res) {
   return guarded([&] {
     if (h.dim() != 3) bad_value("the block input must be (B, L, d_model); got " + shape_str(h));
     variable_list per;
@@ -942,7 +953,7 @@ Tensor directional(const Tensor& h, const std::vector<Tensor>& params, const std
     const bool save = !detach && at::GradMode::is_enabled() && needs;
     const Tensor y = CoreFn::apply(args[0], args[1], args[2], args[3], args[4], args[5], args[6], args[7], tok,
                                    chunk_len, save);                                          // :170-190
-    return out_proj(y, per[8]);                                                              // :191, :562-566
+    return out_proj(y, per[8], res);                                                         // :191, :562-566
   });
 }
 
@@ -976,7 +987,7 @@ PYBIND11_MODULE(_native, m) {
   m.def("conv_silu", &conv_silu);
   m.def("norm", &norm);
   m.def("in_proj", [](const Tensor& h, const Tensor& W) { return guarded([&] { return in_proj(h, W); }); });
-  m.def("out_proj", [](const Tensor& y, const Tensor& W) { return guarded([&] { return out_proj(y, W); }); });
+  m.def("out_proj", [](const Tensor& y, const Tensor& W) { return guarded([&] { return out_proj(y, W, std::nullopt); }); });
   m.def("batched", &batched_py);
   m.def("direction_params", &direction_params);
   m.def("stacks_match", &stacks_match);

@@ -131,7 +131,7 @@ class BidirectionalMambaBlock(nn.Module):
         blocks = [self.forward_mamba, self.backward_mamba]
         if any(_custom_scan(b) for b in blocks):
             return xr + _per_direction_forward(blocks, h, tok)
-        return xr + _directional_forward(blocks, h, tok, self.scan_mode, self, blocks)
+        return _directional_forward(blocks, h, tok, self.scan_mode, self, blocks, residual=xr)
 
 
 class MultiDirectionalMambaBlock(nn.Module):
@@ -174,8 +174,8 @@ class MultiDirectionalMambaBlock(nn.Module):
             blocks = list(self.mamba_blocks)
         if any(_custom_scan(b) for b in blocks):
             return xr + _per_direction_forward(blocks, h, tok)
-        return xr + _directional_forward(blocks, h, tok, self.scan_mode, self,
-                                         list(self.mamba_blocks))                # :562-566
+        return _directional_forward(blocks, h, tok, self.scan_mode, self,
+                                    list(self.mamba_blocks), residual=xr)         # :562-566
 
 
 # per-direction parameters stored as slices of one (K, ...) buffer per kind
@@ -299,9 +299,10 @@ def _per_direction_forward(blocks, h, tok):
     return y
 
 
-def _directional_forward(blocks, h, tok, scan_mode, owner=None, stacked=None):
+def _directional_forward(blocks, h, tok, scan_mode, owner=None, stacked=None, residual=None):
     """Run len(blocks) MambaBlocks on one (B, N, E) input, block k scanning
-    in the order of tok[k], and return the sum of their outputs.  The
+    in the order of tok[k], and return the sum of their outputs and of the
+    ``residual``, which out_proj's product adds as it stores.  The
     parameters of ``stacked`` (all direction blocks of ``owner``, of which
     ``blocks`` are the first) are slices of one buffer per kind; without an
     owner there is one block, whose parameters are used as they are."""
@@ -314,4 +315,5 @@ def _directional_forward(blocks, h, tok, scan_mode, owner=None, stacked=None):
     flat = [p for ps in params for p in ps[:K]]
     chunk_len = _resolve_chunk(h.shape[1], mode_chunk_len(scan_mode))
     # the reference's "metal" mode is inference only (mamba_metal.py:230)
-    return _lib.native().directional(h, flat, stacks, K, tok, chunk_len, scan_mode == "metal")
+    return _lib.native().directional(h, flat, stacks, K, tok, chunk_len, scan_mode == "metal",
+                                     residual)

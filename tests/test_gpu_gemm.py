@@ -29,11 +29,12 @@ def _operand(rows, k, kmajor, batch, pad, gen):
     return (v if kmajor else v.transpose(1, 2)), buf, ld, r * ld
 
 
-def _run(desc, A, B, C):
+def _run(desc, A, B, C, add=None):
     lib = _lib.lib()
     nbytes = _lib.check(lib.mvm_gemm_workspace_bytes(ctypes.byref(desc)))
     ws = torch.full((max(nbytes, 1),), 255, dtype=torch.uint8, device="cuda")  # NaN if read before written
-    _lib.check(lib.mvm_gemm_f32(ctypes.byref(desc), A.data_ptr(), B.data_ptr(), C.data_ptr(), ws.data_ptr(),
+    _lib.check(lib.mvm_gemm_f32(ctypes.byref(desc), A.data_ptr(), B.data_ptr(),
+                                add.data_ptr() if add is not None else None, C.data_ptr(), ws.data_ptr(),
                                 nbytes, torch.cuda.current_stream().cuda_stream))
 
 
@@ -54,19 +55,20 @@ def test_product(cuda, m, n, k, batch, splits, pad, akm, bkm):
     a, A, lda, sa = _operand(m, max(k, 1), akm, batch, pad, gen)
     b, B, ldb, sb = _operand(n, max(k, 1), bkm, batch, pad, gen)
     ldc = n + 3
-    for acc in (0, 1):
+    for acc in (0, 1, 2):  # nothing, C itself, another buffer is added
         C0 = torch.randn(batch, m, ldc, generator=gen).cuda()
-        C = C0.clone()
-        d = _lib.GemmDesc(m, n, k, batch, lda, ldb, ldc, sa, sb, m * ldc, 0, 0, akm, bkm, acc, splits)
-        _run(d, A, B, C)
+        C = C0.clone() if acc < 2 else torch.randn(batch, m, ldc, generator=gen).cuda()
+        keep = C.clone()
+        d = _lib.GemmDesc(m, n, k, batch, lda, ldb, ldc, sa, sb, m * ldc, 0, 0, akm, bkm, 0, splits)
+        _run(d, A, B, C, (None, C, C0)[acc])
         ad, bd = a.double()[:, :, :k], b.double()[:, :, :k].transpose(1, 2).contiguous()
         ref = ad @ bd + (C0.double()[:, :, :n] if acc else 0)
         S = ad.abs() @ bd.abs() + (C0.double()[:, :, :n].abs() if acc else 0)
         bound = (6 * -(-k // 16) + max(splits, 24) + 2) * 2.0 ** -23 * S
         assert ((C.double()[:, :, :n] - ref).abs() <= bound).all()
-        assert torch.equal(C[:, :, n:], C0[:, :, n:])  # nothing outside the matrix
-        again = C0.clone()
-        _run(d, A, B, again)
+        assert torch.equal(C[:, :, n:], keep[:, :, n:])  # nothing outside the matrix
+        again = keep.clone()
+        _run(d, A, B, again, (None, again, C0)[acc])
         assert torch.equal(again, C)
 
 
