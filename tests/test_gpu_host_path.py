@@ -1,0 +1,123 @@
+"""The C++ host path (csrc/torch_ext.cpp): what its autograd Functions have
+to keep besides the numbers the other tests check -- saved-tensor hooks,
+streams, in-place checks, error types, launch timing, and the carry passes at
+the edges of their batches."""
+
+import numpy as np
+import pytest
+import torch
+
+import mlx_vision_mamba_amd as mvm
+from mlx_vision_mamba_amd import _lib, scan, synthetic
+from oracle import ref_lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(cuda):
+    torch.manual_seed(0)
+    m = mvm.MultiDirectionalMambaBlock(32, d_state=4, num_directions=4, grid_shape=(4, 5), scan_mode="hip").to(cuda)
+    x = torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(1)).to(cuda).requires_grad_()
+    g = torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(2)).to(cuda)
+    return m, x, g
+
+
+def _step(m, x, g):
+    y = m(x)
+    return [y.detach(), *torch.autograd.grad(y, [x, *m.parameters()], g)]
+
+
+def test_saved_tensor_hooks_and_side_stream(cuda):
+    """The same results with every saved tensor moved to the host and back
+    between forward and backward, and on another stream."""
+    m, x, g = _block(cuda)
+    ref = _step(m, x, g)
+    seen = []
+
+    def pack(t):
+        seen.append(tuple(t.shape))
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(cuda)):
+        got = _step(m, x, g)
+    assert len(seen) >= 14
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        got = _step(m, x, g)
+    torch.cuda.current_stream().wait_stream(s)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
+def test_inplace_change_of_a_saved_input_raises(cuda):
+    u, dl, A, Bm, Cm, Dv, g = [t.to(cuda) for t in synthetic.make(1, 20, 8, 4, seed=0)]
+    u.requires_grad_()
+    y = scan.selective_scan(u, dl, A, Bm, Cm, Dv)
+    dl.add_(0.1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward(g)
+
+
+def test_no_checkpoints_without_a_gradient(cuda):
+    """Under no_grad, and for inputs that need no gradient, nothing is kept."""
+    u, dl, A, Bm, Cm, Dv, _ = [t.to(cuda) for t in synthetic.make(1, 20, 8, 4, seed=0)]
+    assert scan.selective_scan(u, dl, A, Bm, Cm, Dv).grad_fn is None
+    with torch.no_grad():
+        assert scan.selective_scan(u.requires_grad_(), dl, A, Bm, Cm, Dv).grad_fn is None
+    assert not scan.selective_scan_metal(u, dl, A, Bm, Cm, Dv).requires_grad
+    assert scan.selective_scan(u, dl, A, Bm, Cm, Dv).grad_fn is not None
+
+
+def test_error_types(cuda):
+    """Library refusals stay ScanError with their code, bad shapes ValueError,
+    tensors elsewhere RuntimeError."""
+    K = 65536
+    u, A = torch.zeros(1, 1, K, 1, device=cuda), torch.zeros(K, 1, 1, device=cuda)
+    with pytest.raises(_lib.ScanError) as e:
+        scan.scan_forward(u, u, A, u, u, torch.zeros(K, 1, device=cuda))
+    assert e.value.code == _lib.MVM_ERR_UNSUPPORTED and "65535" in str(e.value)
+    x = torch.zeros(1, 4, 8, device=cuda)
+    with pytest.raises(ValueError, match="d_state"):
+        scan.selective_scan(x, x, torch.zeros(8, 17, device=cuda), torch.zeros(1, 4, 17, device=cuda),
+                            torch.zeros(1, 4, 17, device=cuda), torch.zeros(8, device=cuda))
+    with pytest.raises(ValueError, match="B and C"):
+        scan.selective_scan(x, x, torch.zeros(8, 2, device=cuda), torch.zeros(1, 4, 3, device=cuda),
+                            torch.zeros(1, 4, 2, device=cuda), torch.zeros(8, device=cuda))
+    with pytest.raises(RuntimeError, match="must be on"):
+        scan.selective_scan(x, x, torch.zeros(8, 2), torch.zeros(1, 4, 2, device=cuda),
+                            torch.zeros(1, 4, 2, device=cuda), torch.zeros(8, device=cuda))
+
+
+def test_launch_timing_records(cuda):
+    m, x, g = _block(cuda)
+    rec = []
+    scan.set_scan_timing(rec)
+    try:
+        _step(m, x, g)
+    finally:
+        scan.set_scan_timing(None)
+    _step(m, x, g)
+    torch.cuda.synchronize()
+    assert [r[0] for r in rec] == ["fwd", "bwd"]
+    f, b = scan.algorithmic_bytes_fused(2 * 4, 20, 64, 4, 4)
+    assert [r[3] for r in rec] == [f, b] and all(r[1].elapsed_time(r[2]) > 0 for r in rec)
+
+
+@pytest.mark.parametrize("nchunk", [9, 16, 17, 24, 25])
+def test_carry_batches(cuda, nchunk):
+    """The carry passes load 8 chunks at a time: chunk counts at the edges of
+    the batches (the last chunk partial) against the float64 oracle."""
+    L = 16 * nchunk - 5
+    ins = synthetic.make(2, L, 40, 16, seed=nchunk)
+    t = [v.to(cuda) for v in ins]
+    u4, d4, A3, B4, C4, D2 = t[0][:, :, None], t[1][:, :, None], t[2][None], t[3][:, :, None], t[4][:, :, None], t[5][None]
+    y, ck = scan.scan_forward(u4, d4, A3, B4, C4, D2, chunk_len=16, save_ckpt=True)
+    got = [y, *scan.scan_backward(u4, d4, A3, B4, C4, D2, t[6][:, :, None], ck, chunk_len=16)]
+    np_in = [v.numpy() for v in ins]
+    refs = [ref_lib.scan_fwd(*np_in[:6])] + list(ref_lib.scan_vjp(*np_in))
+    for name, a, r in zip(["y", "du", "ddelta", "dA", "dB", "dC", "dD"], got, refs):
+        a = a.double().cpu().numpy().reshape(r.shape)
+        assert (np.abs(a - r) <= 1e-5 + 1e-4 * np.abs(r)).all(), name
