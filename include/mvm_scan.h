@@ -215,6 +215,18 @@ int mvm_scan_fused_fwd(const mvm_scan_fused_desc* desc, const float* u, const fl
                        float* y_raw, float* ckpt, void* workspace, size_t workspace_bytes,
                        void* stream);
 
+/* mvm_scan_fused_fwd with delta_raw = dt @ W_dt^T formed inside
+ * (mamba_block.py:180): dt holds dt_rank columns (1..MVM_SCAN_MAX_DT_RANK) in
+ * rows of the B-like strides, W_dt is (ndir, dim, dt_rank).  delta_raw
+ * (dt_stride_*) is written for the backward, or NULL.  The workspace is that
+ * of mvm_scan_fused_fwd. */
+#define MVM_SCAN_MAX_DT_RANK 48
+int mvm_scan_fused_dt_fwd(const mvm_scan_fused_desc* desc, const float* u, const float* dt,
+                          int32_t dt_rank, const float* W_dt, const float* delta_bias,
+                          const float* A, const float* Bm, const float* Cm, const float* Dv,
+                          const float* z, float* y, float* y_raw, float* delta_raw, float* ckpt,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* VJP of mvm_scan_fused_fwd for upstream dy (gradient of the gated y).
  * ckpt is required; y_raw and dz are required when z is given; ddelta_bias
  * (ndir, dim) is required when delta_bias is given.  ddelta_raw is the

@@ -121,6 +121,8 @@ SIGNATURES = {
     "mvm_scan_fused_validate": (ctypes.c_int, [ctypes.POINTER(FusedDesc)]),
     "mvm_scan_fused_workspace_bytes": (_i64, [ctypes.POINTER(FusedDesc), ctypes.c_int, ctypes.c_int]),
     "mvm_scan_fused_fwd": (ctypes.c_int, [ctypes.POINTER(FusedDesc)] + [_vp] * 12 + [ctypes.c_size_t, _vp]),
+    "mvm_scan_fused_dt_fwd": (ctypes.c_int, [ctypes.POINTER(FusedDesc), _vp, _vp, _i32] + [_vp] * 12
+                              + [ctypes.c_size_t, _vp]),
     "mvm_scan_fused_bwd": (ctypes.c_int, [ctypes.POINTER(FusedDesc)] + [_vp] * 20 + [ctypes.c_size_t, _vp]),
     "mvm_conv_validate": (ctypes.c_int, [ctypes.POINTER(ConvDesc)]),
     "mvm_conv_workspace_bytes": (_i64, [ctypes.POINTER(ConvDesc)]),

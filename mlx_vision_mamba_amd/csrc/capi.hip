@@ -534,6 +534,39 @@ int mvm_scan_fused_fwd(const mvm_scan_fused_desc* desc, const float* u, const fl
                     "mvm_scan_fused_fwd launch");
 }
 
+int mvm_scan_fused_dt_fwd(const mvm_scan_fused_desc* desc, const float* u, const float* dt,
+                          int32_t dt_rank, const float* W_dt, const float* delta_bias,
+                          const float* A, const float* Bm, const float* Cm, const float* Dv,
+                          const float* z, float* y, float* y_raw, float* delta_raw, float* ckpt,
+                          void* workspace, size_t workspace_bytes, void* stream) {
+  static_assert(MVM_SCAN_MAX_DT_RANK == mvm::kDtMaxRank, "header and kernel agree on the dt rank");
+  int rc = check_fused(desc);
+  if (rc != MVM_OK) return rc;
+  if (dt_rank < 1 || dt_rank > mvm::kDtMaxRank)
+    return fail(MVM_ERR_UNSUPPORTED, "dt_rank=%d unsupported (1..%d)", dt_rank, mvm::kDtMaxRank);
+  const mvm::Geom g = fused_geom(desc);
+  const bool empty = g.B == 0 || g.L == 0 || g.D == 0;
+  if (!empty) {
+    if (!u || !dt || !W_dt || !A || !Bm || !Cm || !Dv || !y)
+      return fail(MVM_ERR_INVALID_ARG, "mvm_scan_fused_dt_fwd: NULL input or y pointer");
+    if (g.L > 1 && g.bst < dt_rank)
+      return fail(MVM_ERR_INVALID_ARG, "mvm_scan_fused_dt_fwd: dt rows overlap");
+    if (z && !z_ok(desc)) return fail(MVM_ERR_INVALID_ARG, "mvm_scan_fused_dt_fwd: z strides overlap");
+    if ((reinterpret_cast<uintptr_t>(ckpt) & 15u) != 0)
+      return fail(MVM_ERR_INVALID_ARG, "mvm_scan_fused_dt_fwd: ckpt must be 16-byte aligned");
+  }
+  const FwdWs w = fwd_ws(g);
+  rc = check_ws("mvm_scan_fused_dt_fwd", workspace, workspace_bytes, w.total);
+  if (rc != MVM_OK) return rc;
+  if (empty) return ok();
+  char* ws = static_cast<char*>(workspace);
+  mvm::FwdBufs b{u, nullptr, A, Bm, Cm, Dv, y, ckpt,
+                 reinterpret_cast<float*>(ws), reinterpret_cast<float*>(ws + w.agg_h),
+                 delta_bias, z, y_raw, dt, W_dt, dt_rank, delta_raw};
+  return hip_status(mvm::launch_fused_dt_fwd(g, b, static_cast<hipStream_t>(stream)),
+                    "mvm_scan_fused_dt_fwd launch");
+}
+
 int mvm_scan_fused_bwd(const mvm_scan_fused_desc* desc, const float* u, const float* delta_raw,
                        const float* delta_bias, const float* A, const float* Bm, const float* Cm,
                        const float* Dv, const float* z, const float* y_raw, const float* ckpt,

@@ -31,6 +31,10 @@ constexpr int64_t kFoldMax = 8;
 // chunks whose aggregates a carry pass has in flight together
 constexpr int kCarryBatch = 8;
 
+// largest dt rank whose projection the fused forward forms itself (its LDS
+// rows keep six workgroups on a CU)
+constexpr int kDtMaxRank = 48;
+
 struct bf16_t {
   uint16_t bits;
 };

@@ -53,6 +53,12 @@ struct FwdBufs {
   const float* dbias;  // (K, D) or null (zero bias)
   const float* z;      // gate or null (no gate)
   float* y_raw;        // ungated output or null
+  // fused dt_proj: delta_raw = dt @ W_dt^T formed in the kernel (delta is
+  // then not read); dt has rank columns in rows of the B / C strides
+  const float* dt = nullptr;
+  const float* W_dt = nullptr;  // (K, D, rank)
+  int32_t rank = 0;             // 1..kDtMaxRank
+  float* delta_out = nullptr;   // delta_raw as it is formed, for the backward, or null
 };
 
 struct BwdBufs {
@@ -92,6 +98,8 @@ hipError_t launch_bwd(const Geom& g, const BwdBufs& b, int in_dtype, int out_dty
                       hipStream_t s);
 // fused form (float32 only): softplus(delta_raw + dbias) on load, gate on store
 hipError_t launch_fused_fwd(const Geom& g, const FwdBufs& b, hipStream_t s);
+// the same with dt_proj in the kernel (b.dt, b.W_dt, b.rank)
+hipError_t launch_fused_dt_fwd(const Geom& g, const FwdBufs& b, hipStream_t s);
 hipError_t launch_fused_bwd(const Geom& g, const BwdBufs& b, hipStream_t s);
 hipError_t launch_fill(float* p, int64_t n, float v, hipStream_t s);
 hipError_t launch_selftest_lanes(float* out, hipStream_t s);

@@ -389,9 +389,12 @@ void check_fused(const Tensor& u, const Tensor& delta_raw, const Tensor& dbias, 
 struct FusedOut {
   Tensor y, y_raw, ckpt;
 };
+// delta_raw is read; or, with dt (B, L, K, R) in rows of B's strides and W_dt
+// (K, D, R), formed in the kernel and written to delta_raw when saving
 FusedOut fused_fwd(const Tensor& u, const Tensor& delta_raw, const Tensor& dbias, const Tensor& A,
                    const Tensor& Bm, const Tensor& Cm, const Tensor& Dv, const Tensor& z, const Tensor& tok,
-                   int64_t chunk_len, bool save, bool a_is_log) {
+                   int64_t chunk_len, bool save, bool a_is_log, const Tensor& dt = Tensor(),
+                   const Tensor& W_dt = Tensor()) {
   check_fused(u, delta_raw, dbias, A, Bm, Cm, Dv, z);
   FusedOut o;
   c10::OptionalDeviceGuard guard(u.device());
@@ -402,9 +405,15 @@ FusedOut fused_fwd(const Tensor& u, const Tensor& delta_raw, const Tensor& dbias
   const int64_t nbytes = check(mvm_scan_fused_workspace_bytes(&f, 0, z.defined()));
   const Tensor ws = workspace(nbytes, u);
   Timed timed("fwd");
-  check(mvm_scan_fused_fwd(&f, fp(u), fp(delta_raw), fp(dbias), fp(A), fp(Bm), fp(Cm), fp(Dv), fp(z), fpm(o.y),
-                           fpm(o.y_raw), fpm(o.ckpt), ws.mutable_data_ptr(), static_cast<size_t>(nbytes),
-                           stream_of(u)));
+  if (dt.defined())
+    check(mvm_scan_fused_dt_fwd(&f, fp(u), fp(dt), static_cast<int32_t>(dt.size(3)), fp(W_dt), fp(dbias), fp(A),
+                                fp(Bm), fp(Cm), fp(Dv), fp(z), fpm(o.y), fpm(o.y_raw),
+                                save ? fpm(delta_raw) : nullptr, fpm(o.ckpt), ws.mutable_data_ptr(),
+                                static_cast<size_t>(nbytes), stream_of(u)));
+  else
+    check(mvm_scan_fused_fwd(&f, fp(u), fp(delta_raw), fp(dbias), fp(A), fp(Bm), fp(Cm), fp(Dv), fp(z), fpm(o.y),
+                             fpm(o.y_raw), fpm(o.ckpt), ws.mutable_data_ptr(), static_cast<size_t>(nbytes),
+                             stream_of(u)));
   const auto nb = fused_bytes(u.size(0) * u.size(2), u.size(1), u.size(3), A.size(-1), u.size(2), z.defined(),
                               dbias.defined());
   timed.stop(nb.first, nb.second);
@@ -628,11 +637,12 @@ mvm_gemm_desc gemm_desc(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ld
 
 constexpr int64_t kMaxLd = int64_t{1} << 21;
 
-// batch x rows from which dt_proj's two products over the rows (delta_raw and
-// its gradient's) are left to the BLAS library: they stream 77 MB at 4 x 6272
-// rows of 768 channels, with almost no arithmetic, and the library's picks
-// take 25.6 and 22.3 us there, the kernels here 31.4 and 27.3; at 8 x 1024
-// rows it is 21 and 20 us against 12.1 and 13.7.
+// batch x rows from which dt_proj's products over the rows (delta_raw's
+// gradient, and delta_raw itself where the scan does not form it) are left to
+// the BLAS library: they stream 77 MB at 4 x 6272 rows of 768 channels, with
+// almost no arithmetic, and the library's picks take 22.3 and 25.6 us there,
+// the kernels here 27.3 and 31.4; at 8 x 1024 rows it is 20 and 21 us against
+// 13.7 and 12.1.
 constexpr int64_t kStreamRows = 16384;
 
 // out[q] (+)= op(A[q]) @ op(B[q]) for float32 (batch, rows, cols) views; ta /
@@ -852,7 +862,8 @@ Tensor padded_rows(int64_t K, int64_t rows, int64_t P, const Tensor& like) {
 // (mamba_block.py:166-190, all K directions at once):
 //   xc    = silu(causal depthwise conv(x) + conv_b)      along each scan order
 //   dbc   = x_proj(xc)                                   (K, B*N, R + 2N)
-//   delta = softplus(dt_proj(dbc[:R]) + dt_bias)         inside the scan
+//   delta = softplus(dt_proj(dbc[:R]) + dt_bias)         inside the scan, dt_proj
+//           included up to rank 48 (d_model 768), and delta_raw written for the backward
 //   y     = scan(xc, delta, -exp(A_log), B, C, D) * silu(z)
 // The scan kernels take A_log and form A = -exp(A_log) themselves; their dA
 // output is the gradient of A_log.  The backward writes the gradient of xz in
@@ -869,11 +880,19 @@ struct CoreFn : Function<CoreFn> {
     conv_fwd(xb, conv_w, conv_b, bnkd(xc, bsz, n), tok);                               // :170-171
     Tensor dbc = padded_rows(K, M, R + 2 * ns, xz);
     batched(xc, W_x, dbc, false, true, false, false);                                  // :174
-    Tensor delta_raw = empty_like_opts({K, M, din}, xz);
-    batched(dbc.narrow(2, 0, R), W_dt, delta_raw, false, true, false, true);           // :180
     const Tensor bc = bnkd(dbc, bsz, n);
+    // dt_proj (:180) inside the scan, up to its largest rank; else, and when
+    // delta_raw of many rows is kept for the backward, as a product (writing
+    // it from the scan costs there what the product does: 4 x 6272 rows
+    // trained 1542 us a block step inside, 1534 with the product; forward
+    // only, 8 x 1024 rows, 1289 us an encoder pass inside, 1314 with it)
+    const bool dt_in = R <= MVM_SCAN_MAX_DT_RANK && W_dt.is_contiguous() && !(save && K * M > kStreamRows);
+    // (forward only: delta_raw is never formed in memory; xc lends its layout)
+    Tensor delta_raw = dt_in && !save ? xc : empty_like_opts({K, M, din}, xz);
+    if (!dt_in) batched(dbc.narrow(2, 0, R), W_dt, delta_raw, false, true, false, true);
     const auto o = fused_fwd(bnkd(xc, bsz, n), bnkd(delta_raw, bsz, n), b_dt, A_log, bc.narrow(3, R, ns),
-                             bc.narrow(3, R + ns, ns), Dv, z, tok, chunk_len, save, true);  // :181-190
+                             bc.narrow(3, R + ns, ns), Dv, z, tok, chunk_len, save, true,
+                             dt_in ? bc.narrow(3, 0, R) : Tensor(), W_dt);                  // :180-190
     if (save) {
       ctx->save_for_backward({xz, conv_w, conv_b, W_x, W_dt, b_dt, A_log, Dv, tok, xc, dbc, delta_raw, o.y_raw,
                               o.ckpt});
