@@ -650,7 +650,14 @@ constexpr int64_t kStreamRows = 16384;
 // rows of an operand whose summed index is the contiguous one (from 32 summed
 // values up); other operands, and `stream` products of many rows, are torch's.
 void batched(const Tensor& A, const Tensor& B, Tensor& out, bool ta, bool tb, bool accumulate, bool stream) {
+  TORCH_CHECK(A.dim() == 3 && B.dim() == 3 && out.dim() == 3, "batched products take 3-D tensors");
   const int64_t q = A.size(0), m = A.size(ta ? 2 : 1), k = A.size(ta ? 1 : 2), n = B.size(tb ? 1 : 2);
+  // (the kernels only see pointers: the checks torch's products would make)
+  TORCH_CHECK(B.size(0) == q && B.size(tb ? 2 : 1) == k && out.sizes() == at::IntArrayRef({q, m, n}),
+              "batched products of ", A.sizes(), " and ", B.sizes(), " into ", out.sizes(), " do not fit");
+  check_device({&A, &B, &out});
+  for (const Tensor* t : {&A, &B, static_cast<const Tensor*>(&out)})
+    TORCH_CHECK(t->scalar_type() == at::kFloat, "batched products take float32; got ", t->scalar_type());
   auto rows16 = [](const Tensor& t) { return t.stride(1) % 4 == 0 && t.stride(0) % 4 == 0 && aligned16(t); };
   const bool ok = A.stride(2) == 1 && B.stride(2) == 1 && out.stride(2) == 1 && A.stride(1) < kMaxLd &&
                   B.stride(1) < kMaxLd && (k < 32 || ((ta || rows16(A)) && (!tb || rows16(B)))) &&
@@ -771,13 +778,13 @@ struct OutProjFn : Function<OutProjFn> {
 };
 
 Tensor in_proj(const Tensor& h, const Tensor& W) {
-  if (usable(h, W, {W.size(0), W.size(1)})) return InProjFn::apply(h, W);
+  if (h.size(-1) == W.size(1) && usable(h, W, {W.size(0), W.size(1)})) return InProjFn::apply(h, W);
   return at::linear(h, W);
 }
 
 Tensor out_proj(const Tensor& y, const Tensor& W, const OptTensor& res) {
   const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
-  if (usable(y, W, {E, D, K * D}) && (K == 1 || D % 16 == 0)) {
+  if (y.size(-1) == D && y.size(-2) == K && usable(y, W, {E, D, K * D}) && (K == 1 || D % 16 == 0)) {
     auto shape = y.sizes().vec();
     shape.pop_back();
     shape.back() = E;
@@ -875,6 +882,11 @@ struct CoreFn : Function<CoreFn> {
     const Tensor tok = tok_.value_or(Tensor());
     const int64_t bsz = xz.size(0), n = xz.size(1), K = xz.size(2), din = xz.size(3) / 2;
     const int64_t R = W_dt.size(2), ns = A_log.size(2), M = bsz * n;
+    check_device({&xz, &conv_w, &conv_b, &W_x, &W_dt, &b_dt, &A_log, &Dv});
+    TORCH_CHECK(conv_w.size(0) == K && conv_w.size(1) == din && conv_b.sizes() == at::IntArrayRef({K, din}) &&
+                    W_dt.sizes() == at::IntArrayRef({K, din, R}),
+                "the block's conv ", conv_w.sizes(), ", ", conv_b.sizes(), " and dt_proj ", W_dt.sizes(),
+                " do not fit K=", K, ", D_inner=", din);
     const Tensor xb = xz.narrow(3, 0, din), z = xz.narrow(3, din, din);
     Tensor xc = empty_like_opts({K, M, din}, xz);
     conv_fwd(xb, conv_w, conv_b, bnkd(xc, bsz, n), tok);                               // :170-171

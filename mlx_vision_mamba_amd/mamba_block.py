@@ -228,7 +228,8 @@ def _direction_stacks(owner, blocks):
 def _stacks_of(owner, params):
     flat = [p for ps in params for p in ps]
     bufs = owner.__dict__.get("_param_stacks")
-    if bufs is not None and _lib.native().stacks_match(bufs, flat):
+    # (a module pickled by an older version holds a tuple here)
+    if isinstance(bufs, list) and _lib.native().stacks_match(bufs, flat):
         return bufs
     with torch.no_grad():
         bufs = [torch.stack([p.detach() for p in ps], 0) for ps in params]

@@ -1,12 +1,15 @@
-"""Host-side checks of include/mvm_gemm.h (no GPU, no launches)."""
+"""Host-side checks of include/mvm_gemm.h and of the products and parameter
+buffers of csrc/torch_ext.cpp (no GPU, no launches)."""
 
 import ctypes
 import os
 import re
 
 import pytest
+import torch
 
-from mlx_vision_mamba_amd import _lib
+import mlx_vision_mamba_amd as mvm
+from mlx_vision_mamba_amd import _lib, gemm, mamba_block
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -49,3 +52,32 @@ def test_workspace_is_the_split():
     assert ws(splits=3) == 3 * 64 * 4
     n = ws(m=6272, n=384, k=6144, lda=6144, ldb=6144, ldc=384)
     assert n > 0 and n % (6272 * 384 * 4) == 0
+
+
+@pytest.mark.parametrize("a,b,out,ta,tb,what", [
+    ((2, 6, 8), (2, 4, 7), None, False, True, "do not fit"),       # summed lengths differ
+    ((2, 6, 8), (3, 8, 4), None, False, False, "do not fit"),      # batches differ
+    ((2, 8, 6), (2, 8, 4), (2, 6, 5), True, False, "do not fit"),  # output columns
+    ((6, 8), (2, 8, 4), None, False, False, "3-D|out of range"),
+    ((2, 6, 8), (2, 8, 4), None, False, False, "only on the GPU"),
+])
+def test_batched_products_refuse_operands_that_do_not_fit(a, b, out, ta, tb, what):
+    """The kernels see pointers only, so the host refuses what torch's
+    batched product would refuse (and CPU tensors: there is no fallback)."""
+    with pytest.raises((RuntimeError, IndexError), match=what):
+        gemm.batched(torch.zeros(a), torch.zeros(b), None if out is None else torch.zeros(out), ta=ta, tb=tb)
+
+
+def test_stacks_of_an_older_pickle_are_rebuilt():
+    """A direction module pickled whole by an older version holds a (buffers,
+    pointers) tuple where the buffers are now: rebuilt, values kept."""
+    m = mvm.BidirectionalMambaBlock(8, d_state=2, scan_mode="hip")
+    blocks = [m.forward_mamba, m.backward_mamba]
+    before = {k: v.clone() for k, v in m.state_dict().items()}
+    bufs = mamba_block._direction_stacks(m, blocks)
+    assert mamba_block._direction_stacks(m, blocks) is bufs
+    m.__dict__["_param_stacks"] = (bufs, [(0, torch.float32, (1,))])
+    again = mamba_block._direction_stacks(m, blocks)
+    assert isinstance(again, list) and mamba_block._direction_stacks(m, blocks) is again
+    for k, v in m.state_dict().items():
+        assert torch.equal(v, before[k])

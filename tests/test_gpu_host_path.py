@@ -91,6 +91,26 @@ def test_error_types(cuda):
                             torch.zeros(1, 4, 2, device=cuda), torch.zeros(8, device=cuda))
 
 
+@pytest.mark.parametrize("name", ["conv1d", "x_proj", "dt_proj", "in_proj", "out_proj"])
+def test_block_refuses_parameters_that_do_not_fit(cuda, name):
+    """A submodule left on the CPU, or replaced by one of another width, is
+    an error of the host before anything of it is read on the GPU."""
+    blk = mvm.MambaBlock(32, d_state=4, scan_mode="hip").to(cuda)
+    x = torch.zeros(1, 8, 32, device=cuda)
+    getattr(blk, name).to("cpu")
+    with pytest.raises(RuntimeError):
+        blk(x)
+    getattr(blk, name).to(cuda)
+    blk(x)
+    lay = getattr(blk, name)
+    if name == "conv1d":
+        lay.weight = torch.nn.Parameter(torch.zeros(72, *lay.weight.shape[1:], device=cuda))
+    else:
+        lay.weight = torch.nn.Parameter(torch.zeros(lay.weight.shape[0], lay.weight.shape[1] + 4, device=cuda))
+    with pytest.raises((RuntimeError, ValueError)):
+        blk(x)
+
+
 def test_launch_timing_records(cuda):
     m, x, g = _block(cuda)
     rec = []
