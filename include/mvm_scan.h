@@ -115,7 +115,8 @@ int64_t mvm_scan_ckpt_elems(const mvm_scan_desc* desc);
  * workspace).  Returns < 0 on a bad desc. */
 int64_t mvm_scan_workspace_bytes(const mvm_scan_desc* desc, int which);
 
-/* Time-chunk length the library will use for this descriptor. */
+/* Time-chunk length the library will use for this descriptor (mvm_scan_fwd
+ * without checkpoints and with bf16 results may take longer chunks). */
 int64_t mvm_scan_chunk_len(const mvm_scan_desc* desc);
 
 /* Forward scan.  y may be NULL (checkpoints only); ckpt may be NULL
@@ -204,6 +205,9 @@ int mvm_scan_fused_validate(const mvm_scan_fused_desc* desc);
  * (which = 1); gate != 0 when z is given.  Checkpoints are sized by
  * mvm_scan_ckpt_elems(&desc->scan). */
 int64_t mvm_scan_fused_workspace_bytes(const mvm_scan_fused_desc* desc, int which, int gate);
+
+/* Time-chunk length the fused scans will use for this descriptor. */
+int64_t mvm_scan_fused_chunk_len(const mvm_scan_fused_desc* desc);
 
 /* y = scan(u, softplus(delta_raw + delta_bias), A, Bm, Cm, Dv) * silu(z).
  * delta_bias (ndir, dim) may be NULL (zero bias); z may be NULL (no gate,

@@ -119,6 +119,7 @@ SIGNATURES = {
     "mvm_scan_noalloc_scratch_bytes": (_i64, []),
     "mvm_scan_bwd_noalloc": (ctypes.c_int, [ctypes.POINTER(ScanDesc)] + [_vp] * 15),
     "mvm_scan_fused_validate": (ctypes.c_int, [ctypes.POINTER(FusedDesc)]),
+    "mvm_scan_fused_chunk_len": (_i64, [ctypes.POINTER(FusedDesc)]),
     "mvm_scan_fused_workspace_bytes": (_i64, [ctypes.POINTER(FusedDesc), ctypes.c_int, ctypes.c_int]),
     "mvm_scan_fused_fwd": (ctypes.c_int, [ctypes.POINTER(FusedDesc)] + [_vp] * 12 + [ctypes.c_size_t, _vp]),
     "mvm_scan_fused_dt_fwd": (ctypes.c_int, [ctypes.POINTER(FusedDesc), _vp, _vp, _i32] + [_vp] * 12

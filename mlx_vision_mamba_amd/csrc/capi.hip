@@ -52,22 +52,36 @@ constexpr int64_t kMaxSeqlen = INT32_MAX - 64;
 // Time-chunk length.  One chunk (no carry passes) when the (batch x
 // direction x channel-block) grid alone gives >= 4096 waves (four per SIMD
 // on the 256-CU MI355X); otherwise the sequence is cut until the main passes
-// launch ~16k waves, but into chunks of at least 4 tiles (64 positions) while
-// those give 2048 waves, of 3 tiles while those give 1536, and of 2 below: a
-// shorter chunk repeats more of the per-chunk work (prologue, aggregates,
-// carry) than its waves return.  Measured on MI355X, forward + VJP us by
-// positions per chunk: B=3 L=1037 D=1000: 32 111, 64 103, 96 113; B=16 L=512
-// D=768: 32 174, 48 168, 64 156 (8 chunks: folded without a carry pass);
-// B=1 L=4096 D=768: 32 128, 64 109; B=30 L=300 D=300: 32 106, 64 93; B=10
-// L=331 D=400: 32 68, 48 60 (7 chunks), 64 69; B=2 L=196 D=1536: 32 44, 48 46,
-// 64 54; B=32 L=196 D=3072 is fastest unchunked; B=8 L=16384 D=1536 flat over
-// 256-1024.
-int64_t pick_chunk_len(const mvm_scan_desc* d) {
+// launch ~16k waves, into chunks of at least 2 tiles (32 positions).  With
+// `longer`, chunks have at least 4 tiles (64 positions) while those give 2048
+// waves, 3 tiles while those give 1536, and 2 below: a shorter chunk repeats
+// more of the per-chunk work (prologue, aggregates, carry) than its waves
+// return.  Measured on MI355X, forward + VJP us by positions per chunk: B=3
+// L=1037 D=1000: 32 111, 64 103, 96 113 (bf16 forward alone: 32 43, 64 36);
+// B=16 L=512 D=768: 32 174, 48 168, 64 156 (8 chunks: folded without a carry
+// pass); B=1 L=4096 D=768: 32 128, 64 109; B=30 L=300 D=300: 32 106, 64 93;
+// B=10 L=331 D=400: 32 68, 48 60 (7 chunks), 64 69; B=2 L=196 D=1536: 32 44,
+// 48 46, 64 54; B=32 L=196 D=3072 is fastest unchunked; B=8 L=16384 D=1536
+// flat over 256-1024.
+//
+// Each chunk starts from a carry that one exponential brings over, so the
+// float32 rounding of the recurrence builds up within a chunk only: against 64
+// bits dA is off by 2.3e-7 at 32 positions, 3.1e-7 at 64 and 4.1e-7 unchunked
+// (B=16 L=512 D=768), y by 3.3e-8, 3.5e-8 and 3.6e-8.  So `longer` is for calls
+// whose results do not show it: bf16 forwards without checkpoints (their
+// rounding is 1.7e-3) and the fused scan, where the block's products decide
+// (all gradients of blocks of L=331 and 512 are off by 2-4.6e-7, A_log's by
+// 3.0-3.6e-7).
+int64_t pick_chunk_len(const mvm_scan_desc* d, bool longer) {
   if (d->chunk_len > 0) return d->chunk_len;
   const int64_t tiles = ceil_div(d->seqlen, mvm::kSub);
   const int64_t waves = d->batch * d->ndir * ceil_div(d->dim, mvm::kChPerBlock) * 4;
   int64_t nchunk = 1;
   if (waves < 4096) nchunk = ceil_div(16384, std::max<int64_t>(waves, 1));
+  if (!longer) {
+    nchunk = std::min(nchunk, std::max<int64_t>(1, (tiles + 1) / 2));
+    return std::max<int64_t>(1, ceil_div(tiles, nchunk)) * mvm::kSub;
+  }
   const int64_t least = waves * ceil_div(tiles, 4) >= 2048 ? 4 : (waves * ceil_div(tiles, 3) >= 1536 ? 3 : 2);
   const int64_t tiles_per_chunk = nchunk == 1 ? tiles : std::max(least, ceil_div(tiles, nchunk));
   return std::max<int64_t>(1, tiles_per_chunk) * mvm::kSub;
@@ -129,7 +143,7 @@ int check_desc(const mvm_scan_desc* d) {
   if (d->batch * d->ndir > 65535)
     return fail(MVM_ERR_UNSUPPORTED, "batch*ndir=%lld exceeds 65535",
                 (long long)(d->batch * d->ndir));
-  if (d->seqlen > 0 && ceil_div(d->seqlen, pick_chunk_len(d)) > 65535)
+  if (d->seqlen > 0 && ceil_div(d->seqlen, pick_chunk_len(d, false)) > 65535)
     return fail(MVM_ERR_UNSUPPORTED, "too many time chunks; raise chunk_len");
   // positions are int32 in the kernels, and a tile's rows are formed as
   // position + up to 63 before they are clamped to seqlen - 1
@@ -139,7 +153,7 @@ int check_desc(const mvm_scan_desc* d) {
   return MVM_OK;
 }
 
-mvm::Geom make_geom(const mvm_scan_desc* d) {
+mvm::Geom make_geom(const mvm_scan_desc* d, bool longer = false) {
   mvm::Geom g;
   g.B = d->batch;
   g.L = d->seqlen;
@@ -158,7 +172,7 @@ mvm::Geom make_geom(const mvm_scan_desc* d) {
   g.bsk = d->bc_stride_k;
   g.bst = d->bc_stride_t;
   g.tok = d->seq_to_tok;
-  g.chunk_len = pick_chunk_len(d);
+  g.chunk_len = pick_chunk_len(d, longer);
   g.nchunk = d->seqlen > 0 ? ceil_div(d->seqlen, g.chunk_len) : 0;
   g.nck = ceil_div(d->seqlen, mvm::kCk);
   g.ncblk = ceil_div(d->dim, mvm::kChPerBlock);
@@ -251,7 +265,8 @@ int mvm_scan_fwd(const mvm_scan_desc* desc, const void* u, const float* delta, c
                  void* workspace, size_t workspace_bytes, void* stream) {
   int rc = check_desc(desc);
   if (rc != MVM_OK) return rc;
-  const mvm::Geom g = make_geom(desc);
+  // (mvm_scan_workspace_bytes sizes for the shorter chunks)
+  const mvm::Geom g = make_geom(desc, ckpt == nullptr && desc->out_dtype == MVM_BF16);
   const bool empty = g.B == 0 || g.L == 0 || g.D == 0;
   if (!empty) {
     if (!u || !delta || !A || !Bm || !Cm || !Dv)
@@ -458,7 +473,7 @@ bool z_ok(const mvm_scan_fused_desc* fd) {
 }
 
 mvm::Geom fused_geom(const mvm_scan_fused_desc* fd) {
-  mvm::Geom g = make_geom(&fd->scan);
+  mvm::Geom g = make_geom(&fd->scan, true);
   g.dsb = fd->dt_stride_b; g.dsk = fd->dt_stride_k; g.dst = fd->dt_stride_t;
   g.ysb = fd->y_stride_b;  g.ysk = fd->y_stride_k;  g.yst = fd->y_stride_t;
   g.zsb = fd->z_stride_b;  g.zsk = fd->z_stride_k;  g.zst = fd->z_stride_t;
@@ -495,6 +510,12 @@ extern "C" {
 int mvm_scan_fused_validate(const mvm_scan_fused_desc* desc) {
   const int rc = check_fused(desc);
   return rc == MVM_OK ? ok() : rc;
+}
+
+int64_t mvm_scan_fused_chunk_len(const mvm_scan_fused_desc* desc) {
+  const int rc = check_fused(desc);
+  if (rc != MVM_OK) return rc;
+  return fused_geom(desc).chunk_len;
 }
 
 int64_t mvm_scan_fused_workspace_bytes(const mvm_scan_fused_desc* desc, int which, int gate) {
