@@ -12,16 +12,17 @@ batch 32 of 224x224x1 images ~ N(0,1), patch 16 -> 196 tokens, embed_dim
 (Kaiming-uniform projections, S4D-real A, dt bias with softplus(bias) in
 [1e-3, 1e-1]); loss = mean of the output features; one step = forward +
 loss + backward + AdamW update (the package's one-launch AdamW,
-mlx_vision_mamba_amd.optim; --torch-adamw for torch's fused AdamW).  The fp32 projection
-GEMMs use the TunableOp picks recorded for this step on MI355X
-(mlx_vision_mamba_amd/tuning/, read-only; --default-gemms for the library
-defaults).  Inputs are resident on the GPU before the
+mlx_vision_mamba_amd.optim; --torch-adamw for torch's fused AdamW).  The fp32
+projections run on the package's products (csrc/gemm.hip); dt_proj's two over
+the rows and the patch embedding use the TunableOp picks recorded for this step
+on MI355X (mlx_vision_mamba_amd/tuning/, read-only; --default-gemms for the
+library defaults).  Inputs are resident on the GPU before the
 timed region; W untimed warm-up steps, then exactly K steps between two
 device synchronisations.  value = images / second.  The step is captured once
 in a HIP graph (after the warm-up) and the K timed steps are K replays of it,
-so the host issues one launch per step instead of ~190 kernels through
-Python and autograd (whose ~7-10 ms per step otherwise approaches the GPU
-time on slower hosts); --eager times the eager loop instead.
+so the host issues one launch per step instead of ~180 kernels through
+autograd (whose ~6-7 ms per step otherwise approaches the GPU time on slower
+hosts); --eager times the eager loop instead.
 
 roofline: the fused scan backward call (the block's scan VJP with the
 softplus and silu-gate gradients inside it; the largest hand-written piece
@@ -283,7 +284,7 @@ def bench_encoder(torch, mvm, scan, name, steps, warmup, device):
             "scan_fwd_ms_per_step": round(t_f * 1e3, 3), "scan_bwd_ms_per_step": round(t_b * 1e3, 3),
             "scan_share_of_eager_step": round((t_f + t_b) / (eager / steps), 3),
             "scan_GBps": round((b_f + b_b) / (t_f + t_b) / 1e9, 1),
-            "scan_chunk_len": int(scan.chunk_len_for(shape[0] * model.num_directions, L, 768))}
+            "scan_chunk_len": int(scan.chunk_len_for(shape[0] * model.num_directions, L, 768, fused=True))}
 
 
 def copy_bandwidth(torch, device, iters=20):

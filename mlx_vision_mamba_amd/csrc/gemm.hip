@@ -40,7 +40,7 @@
 // neighbouring lanes share a bank.
 // Bound: with the MFMAs alone the loop runs at 230-240 TFLOP/s; the
 // split's VALU work (11 instructions per pair of values), the LDS traffic and
-// the global loads take the rest: 143-161 TFLOP/s on in_proj and out_proj of
+// the global loads take the rest: 143-170 TFLOP/s on in_proj and out_proj of
 // 6272-16384 rows, where the BLAS library's float32 kernels reach 95-137.
 // Scheduling barriers and raised wave priority around the MFMAs were both
 // slower (they keep the split's instructions from filling in between).
