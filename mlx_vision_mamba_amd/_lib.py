@@ -136,6 +136,7 @@ SIGNATURES = {
     "mvm_adamw_step": (ctypes.c_int, [ctypes.POINTER(AdamwTensor), _i32, ctypes.POINTER(AdamwHparams),
                                       _vp, _vp, _vp, _vp]),
     "mvm_selftest_lanes": (ctypes.c_int, [_vp, _vp]),
+    "mvm_selftest_dt_columns": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
 }
 
 # symbol -> (restype, argtypes) of include/mvm_gemm.h

@@ -729,6 +729,16 @@ int mvm_conv_silu_bwd(const mvm_conv_desc* desc, const float* x, const float* w,
                     "mvm_conv_silu_bwd launch");
 }
 
+int mvm_selftest_dt_columns(int dt_rank, int* cols) {
+  if (dt_rank < 1 || dt_rank > mvm::kDtMaxRank || !cols)
+    return fail(MVM_ERR_INVALID_ARG, "mvm_selftest_dt_columns: dt_rank=%d or NULL cols", dt_rank);
+  const int groups = (mvm::dt_instance(dt_rank) + 15) / 16;
+  for (int m = 0; m < groups; ++m)
+    for (int n = 0; n < 16; ++n)
+      cols[16 * m + n] = mvm::dt_group(m, dt_rank) + mvm::state_col(n, dt_rank - 16 * m);
+  return 16 * groups;
+}
+
 int mvm_selftest_lanes(float* out, void* stream) {
   if (out == nullptr) return fail(MVM_ERR_INVALID_ARG, "out is NULL");
   return hip_status(mvm::launch_selftest_lanes(out, static_cast<hipStream_t>(stream)), "selftest");

@@ -34,6 +34,16 @@ constexpr int kCarryBatch = 8;
 // largest dt rank whose projection the fused forward forms itself (its LDS
 // rows keep six workgroups on a CU)
 constexpr int kDtMaxRank = 48;
+// the instantiation of the fused forward (its rank, a multiple of 4) that a
+// dt rank runs in
+constexpr int dt_instance(int rank) { return rank <= 16 ? 16 : (rank <= 24 ? 24 : kDtMaxRank); }
+// A dt row is staged in groups of 16 columns; m-th group's first column.  An
+// instantiation has groups that lie past a smaller rank (ranks 25..32 in that
+// of 48): they read the row's first column, which always exists (the row may
+// be `rank` values long and the buffer's last), and are masked to zero.
+__host__ __device__ constexpr int dt_group(int m, int rank) { return 16 * m < rank ? 16 * m : 0; }
+// column that lane n of 16 reads of N state values (lanes past N: the first)
+__host__ __device__ constexpr int state_col(int n, int N) { return n < N ? n : 0; }
 
 struct bf16_t {
   uint16_t bits;
@@ -304,7 +314,7 @@ template <typename T, typename IdxT>
 __device__ __forceinline__ float load_state(const T* __restrict__ p, const TileRows& rows, IdxT st,
                                             int N, int tid) {
   const int q = (tid >> 4) & 3, n = tid & 15;
-  const int nc = n < N ? n : 0;
+  const int nc = state_col(n, N);
   if constexpr (std::is_same<IdxT, int32_t>::value) {
     constexpr uint32_t kSz = static_cast<uint32_t>(sizeof(T));
     const int32_t lo = (q & 1) ? rows.r[1] : rows.r[0];

@@ -131,7 +131,8 @@ scan_fwd_kernel(Geom gm, FwdBufs bf) {
                                       ? bf.delta_out + (b * gm.dsb + k * gm.dsk + ch0) : nullptr;
   auto load_dt = [&](const TileRows& rows, float (&v)[RK > 0 ? kDl : 1]) {
 #pragma unroll
-    for (int m = 0; m < kDl; ++m) v[m] = load_state(dtp + 16 * m, rows, sbc, bf.rank - 16 * m, tid);
+    for (int m = 0; m < kDl; ++m)
+      v[m] = load_state(dtp + dt_group(m, bf.rank), rows, sbc, bf.rank - 16 * m, tid);
   };
   auto store_dt = [&](int buf, const float (&v)[RK > 0 ? kDl : 1]) {
 #pragma unroll
@@ -440,9 +441,11 @@ hipError_t launch_fused_fwd(const Geom& g, const FwdBufs& b, hipStream_t s) {
 }
 
 hipError_t launch_fused_dt_fwd(const Geom& g, const FwdBufs& b, hipStream_t s) {
-  if (b.rank <= 16) return launch_fwd_t<float, float, true, 16>(g, b, s);
-  if (b.rank <= 24) return launch_fwd_t<float, float, true, 24>(g, b, s);
-  return launch_fwd_t<float, float, true, 48>(g, b, s);
+  switch (dt_instance(b.rank)) {
+    case 16: return launch_fwd_t<float, float, true, 16>(g, b, s);
+    case 24: return launch_fwd_t<float, float, true, 24>(g, b, s);
+    default: return launch_fwd_t<float, float, true, kDtMaxRank>(g, b, s);
+  }
 }
 
 }  // namespace mvm

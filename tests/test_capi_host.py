@@ -469,3 +469,16 @@ def test_adamw_cpu_parameters_raise_no_fallback():
     from mlx_vision_mamba_amd.optim import AdamW
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         AdamW([torch.nn.Parameter(torch.zeros(3))])
+
+
+def test_dt_columns_stay_inside_the_row():
+    """The fused dt_proj reads no column past the rank of any rank it takes (a
+    row may be just that long, and the buffer's last), and every one before
+    it in its place."""
+    cols = (ctypes.c_int * 48)()
+    for rank in range(1, 49):
+        n = _lib.check(_lib.lib().mvm_selftest_dt_columns(rank, cols))
+        got = list(cols[:n])
+        assert n >= rank and got[:rank] == list(range(rank))
+        assert max(got) < rank, rank
+    assert _lib.lib().mvm_selftest_dt_columns(49, cols) == _lib.MVM_ERR_INVALID_ARG

@@ -114,3 +114,17 @@ def test_block_against_the_restatement(cuda, E):
         err = np.abs(a.detach().double().cpu().numpy() - r.detach().numpy())
         bound = 1e-4 * r.detach().abs().max().item() + 1e-4 * r.detach().abs().numpy()
         assert (err <= bound).all(), (name, err.max())
+
+
+@pytest.mark.parametrize("E,N", [(400, 1), (400, 3), (432, 2), (480, 1), (512, 1)])
+def test_rows_no_longer_than_the_last_column_group(cuda, E, N):
+    """Ranks 25..32 with rows of x_proj's output of at most 34 values: the
+    third group of 16 columns lies past the rank, and past most of the rows."""
+    torch.manual_seed(E)
+    m = mvm.MambaBlock(E, d_state=N, scan_mode="hip").to(cuda)
+    x = torch.randn(2, 19, E, generator=torch.Generator().manual_seed(1))
+    y = m(x.to(cuda))
+    params = torch_ref.params_from_module(m)
+    ref = torch_ref.mamba_block(params, "", x.double(), d_state=N, d_conv=4).detach()
+    err = (y.detach().double().cpu() - ref).abs()
+    assert (err <= 1e-4 * ref.abs().max() + 1e-4 * ref.abs()).all(), err.max()
