@@ -195,6 +195,42 @@ def native():
     return _native
 
 
+class _TracedCall(torch.autograd.Function):
+    """``fn(*args)`` of the C++ host path as one node of a torch.jit trace.
+
+    The tracer keeps a call of a Python Function as a node that runs it again.
+    Of a C++ Function it sees the at:: calls inside, which for a raw launch is
+    just the allocation of its output: the trace would return memory that
+    nothing has written.  The backward goes through the graph that the call
+    itself has built on aliases of its tensors."""
+
+    @staticmethod
+    def forward(ctx, fn, *args):
+        with torch.enable_grad():
+            args = [a.detach().requires_grad_(need) if isinstance(a, torch.Tensor) else a
+                    for a, need in zip(args, ctx.needs_input_grad[1:])]
+            out = fn(*args)
+        ctx.graph = args, out
+        return tuple(t.detach() for t in out) if isinstance(out, tuple) else out.detach()
+
+    @staticmethod
+    def backward(ctx, *grads):
+        args, out = ctx.graph
+        need = [i for i, a in enumerate(args) if isinstance(a, torch.Tensor) and a.requires_grad]
+        got = torch.autograd.grad(out if isinstance(out, tuple) else (out,), [args[i] for i in need], grads,
+                                  retain_graph=True, create_graph=torch.is_grad_enabled(), allow_unused=True)
+        res = [None] * (1 + len(args))
+        for i, g in zip(need, got):
+            res[1 + i] = g
+        return tuple(res)
+
+
+def call(fn, *args):
+    """``fn(*args)``, through a node that the tracer keeps while one is at
+    work.  ``fn`` is a module-level function over the C++ host path."""
+    return _TracedCall.apply(fn, *args) if torch.jit.is_tracing() else fn(*args)
+
+
 def last_error() -> str:
     return lib().mvm_last_error().decode()
 

@@ -13,6 +13,10 @@ import torch
 from . import _lib
 
 
+def _conv_silu(x, weight, bias, tok):
+    return _lib.native().conv_silu(x, weight, bias, tok)
+
+
 def causal_conv_silu(x, weight, bias, seq_to_tok=None):
     """silu(causal depthwise conv) per direction.
 
@@ -28,4 +32,4 @@ def causal_conv_silu(x, weight, bias, seq_to_tok=None):
         if seq_to_tok.dtype != torch.int32 or seq_to_tok.shape != (x.shape[2], x.shape[1]):
             raise ValueError("seq_to_tok must be int32 of shape (K, N)")
         seq_to_tok = seq_to_tok.to(x.device).contiguous()
-    return _lib.native().conv_silu(x, weight, bias, seq_to_tok)
+    return _lib.call(_conv_silu, x, weight, bias, seq_to_tok)

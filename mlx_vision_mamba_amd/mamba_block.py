@@ -314,7 +314,11 @@ def _directional_forward(blocks, h, tok, scan_mode, owner=None, stacked=None, re
         params = _params_of(stacked)
         stacks = _stacks_of(owner, params)
     flat = [p for ps in params for p in ps[:K]]
-    chunk_len = _resolve_chunk(h.shape[1], mode_chunk_len(scan_mode))
     # the reference's "metal" mode is inference only (mamba_metal.py:230)
-    return _lib.native().directional(h, flat, stacks, K, tok, chunk_len, scan_mode == "metal",
-                                     residual)
+    return _lib.call(_directional, h, residual, tok, K, mode_chunk_len(scan_mode), scan_mode == "metal",
+                     len(flat), *flat, *stacks)
+
+
+def _directional(h, residual, tok, K, chunk_len, detach, nparam, *tensors):
+    return _lib.native().directional(h, list(tensors[:nparam]), list(tensors[nparam:]), K, tok,
+                                     _resolve_chunk(h.shape[1], chunk_len), detach, residual)

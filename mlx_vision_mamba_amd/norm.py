@@ -21,13 +21,17 @@ import torch
 from . import _lib
 
 
+def _norm(x, weight, bias, eps, residual):
+    out = _lib.native().norm(x, weight, bias, eps, residual)
+    return tuple(out) if residual else out[0]
+
+
 class _LayerNormFn:
     """The LayerNorm's autograd Function (csrc/torch_ext.cpp)."""
 
     @staticmethod
     def apply(x, weight, bias, eps, residual):
-        out = _lib.native().norm(x, weight, bias, eps, residual)
-        return tuple(out) if residual else out[0]
+        return _lib.call(_norm, x, weight, bias, eps, residual)
 
 
 def layer_norm(x, norm, residual=False):

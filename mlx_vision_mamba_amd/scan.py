@@ -232,14 +232,17 @@ def selective_scan_directions(u, delta, A, B, C, D, seq_to_tok=None, chunk_len=0
         y, _ = scan_forward(u.detach(), delta.detach(), A.detach(), B.detach(), C.detach(),
                             D.detach(), seq_to_tok, _resolve_chunk(u.shape[1], chunk_len), out_dtype)
         return y
-    return _lib.native().scan(u, delta, A, B, C, D, seq_to_tok, _resolve_chunk(u.shape[1], chunk_len), out_dtype,
-                              False)
+    return _lib.call(_scan, u, delta, A, B, C, D, seq_to_tok, chunk_len, out_dtype, False)
+
+
+def _scan(u, delta, A, B, C, D, tok, chunk_len, out_dtype, flat):
+    return _lib.native().scan(u, delta, A, B, C, D, tok, _resolve_chunk(u.shape[1], chunk_len), out_dtype, flat)
 
 
 def _scan3(x, delta, A, B, C, D, chunk_len, out_dtype=None):
     if x.dim() != 3:
         raise ValueError(f"x must be (B, L, D); got {tuple(x.shape)}")
-    return _lib.native().scan(x, delta, A, B, C, D, None, _resolve_chunk(x.shape[1], chunk_len), out_dtype, True)
+    return _lib.call(_scan, x, delta, A, B, C, D, None, chunk_len, out_dtype, True)
 
 
 def selective_scan(x, delta, A, B, C, D, chunk_len=0, out_dtype=None):

@@ -9,6 +9,8 @@ import torch
 
 import mlx_vision_mamba_amd as mvm
 from mlx_vision_mamba_amd import _lib, scan, synthetic
+from mlx_vision_mamba_amd.conv import causal_conv_silu
+from mlx_vision_mamba_amd.norm import layer_norm
 from oracle import ref_lib
 
 pytestmark = pytest.mark.gpu
@@ -158,3 +160,62 @@ def test_bf16_forward_alone_takes_longer_chunks(cuda, bsz, L, D):
     for y in (alone, trained.detach()):
         assert y.dtype == torch.bfloat16
         assert (np.abs(y.double().cpu().numpy() - ref) <= 1e-5 + (2.0 ** -8 + 1e-4) * np.abs(ref)).all()
+
+
+class _Norm(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.n = torch.nn.LayerNorm(32)
+
+    def forward(self, x):
+        h, xr = layer_norm(x, self.n, residual=True)
+        return h * 2 + xr
+
+
+class _Conv(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.w = torch.nn.Parameter(torch.randn(1, 32, 4, generator=torch.Generator().manual_seed(3)))
+        self.b = torch.nn.Parameter(torch.zeros(1, 32))
+
+    def forward(self, x):
+        return causal_conv_silu(x.unsqueeze(2), self.w, self.b)
+
+
+class _Scan(torch.nn.Module):
+    def __init__(self, seed=4):
+        super().__init__()
+        ins = synthetic.make(2, 20, 32, 4, seed=seed)
+        self.p = torch.nn.ParameterList([torch.nn.Parameter(t) for t in ins[2:6]])
+
+    def forward(self, x):
+        A, B, C, D = self.p
+        return scan.selective_scan(x, x.abs(), A, B, C, D)
+
+
+@pytest.mark.parametrize("make", [
+    lambda: mvm.MambaBlock(32, d_state=4, scan_mode="hip"),
+    lambda: mvm.MambaBlock(32, d_state=4, scan_mode="sequential"),
+    lambda: mvm.ResidualMambaBlock(32, d_state=4, scan_mode="hip"),
+    lambda: mvm.BidirectionalMambaBlock(32, d_state=4, scan_mode="hip"),
+    lambda: mvm.MultiDirectionalMambaBlock(32, d_state=4, num_directions=4, grid_shape=(4, 5), scan_mode="hip"),
+    _Norm, _Conv, _Scan], ids=["mamba", "sequential", "residual", "bidirectional", "multi", "norm", "conv", "scan"])
+def test_traced_modules_compute(cuda, make):
+    """A torch.jit trace runs the calls again on new inputs, with and without
+    gradients: the same outputs and gradients as the module's own."""
+    torch.manual_seed(0)
+    m = make().to(cuda)
+    rn = lambda seed: torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(seed)).to(cuda)  # noqa: E731
+    m(rn(0))  # (builds the parameter buffers)
+    t = torch.jit.trace(m, rn(0))
+    x = rn(1).requires_grad_()
+    y, r = t(x), m(x)
+    assert torch.equal(y, r)
+    g = torch.randn(r.shape, generator=torch.Generator().manual_seed(2)).to(cuda)
+    ps = [x, *m.parameters()]
+    for _ in range(2):
+        for a, b in zip(torch.autograd.grad(y, ps, g, retain_graph=True), torch.autograd.grad(r, ps, g, retain_graph=True)):
+            assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(t(x), m(x))
+        assert t(x).grad_fn is None
