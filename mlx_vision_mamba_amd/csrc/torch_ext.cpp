@@ -12,6 +12,7 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
 #include <atomic>
@@ -113,6 +114,27 @@ bool no_overlap(const Tensor& t) {
 }
 
 bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15u) == 0; }
+
+// The gradients `out` of a Function whose backward is raw launches, as they
+// leave it.  Under create_graph they would have no history, and a derivative
+// through them would silently lack this Function's part: they get a node that
+// raises instead, on the paths to the Function's inputs and to the incoming
+// gradients.  (The gradients themselves are right and may be used.)
+variable_list once_differentiable(variable_list out, const variable_list& grads, const char* what) {
+  if (!at::GradMode::is_enabled()) return out;
+  auto edges = torch::autograd::collect_next_edges(grads);
+  if (const auto node = torch::autograd::get_current_node())
+    for (const auto& e : node->next_edges())
+      if (e.is_valid()) edges.push_back(e);
+  const auto err = std::make_shared<torch::autograd::Error>(std::string(what) + " is not twice differentiable",
+                                                            std::move(edges));
+  for (Tensor& t : out)
+    if (t.defined()) {
+      t = t.detach();
+      torch::autograd::create_gradient_edge(t, err);
+    }
+  return out;
+}
 
 // -------------------------------------------------------- launch timing
 //
@@ -304,16 +326,20 @@ struct ScanFn : Function<ScanFn> {
     const auto sv = ctx->get_saved_variables();
     const bool flat = ctx->saved_data["flat"].toBool();
     const int64_t od = ctx->saved_data["out"].toInt();
-    const auto t = lift({sv[0], sv[1], sv[2], sv[3], sv[4], sv[5]}, flat);
-    auto out = scan_bwd(prepare(t[0], t[1], t[2], t[3], t[4], t[5]), flat ? g[0].unsqueeze(2) : g[0], sv[6], sv[7],
-                        ctx->saved_data["chunk"].toInt(),
-                        od < 0 ? std::nullopt : std::make_optional(static_cast<at::ScalarType>(od)));
-    for (int i = 0; i < 6; ++i) {
-      out[i] = out[i].to(sv[i].scalar_type());
-      if (flat) out[i] = out[i].squeeze(i == 2 || i == 5 ? 0 : 2);
+    variable_list out;
+    {
+      at::NoGradGuard no_grad;
+      const auto t = lift({sv[0], sv[1], sv[2], sv[3], sv[4], sv[5]}, flat);
+      out = scan_bwd(prepare(t[0], t[1], t[2], t[3], t[4], t[5]), flat ? g[0].unsqueeze(2) : g[0], sv[6], sv[7],
+                     ctx->saved_data["chunk"].toInt(),
+                     od < 0 ? std::nullopt : std::make_optional(static_cast<at::ScalarType>(od)));
+      for (int i = 0; i < 6; ++i) {
+        out[i] = out[i].to(sv[i].scalar_type());
+        if (flat) out[i] = out[i].squeeze(i == 2 || i == 5 ? 0 : 2);
+      }
     }
     out.resize(11);
-    return out;
+    return once_differentiable(std::move(out), g, "the selective scan");
   }
 };
 
@@ -551,10 +577,15 @@ struct ConvFn : Function<ConvFn> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto sv = ctx->get_saved_variables();
-    const Tensor dy = g[0].to(at::kFloat).contiguous();
-    Tensor dx = empty_like_opts(sv[0].sizes(), sv[0]);
-    auto [dw, db] = conv_bwd(sv[0], sv[1], sv[2], dy, dx, sv[3]);
-    return {dx, dw, db, Tensor()};
+    variable_list out;
+    {
+      at::NoGradGuard no_grad;
+      const Tensor dy = g[0].to(at::kFloat).contiguous();
+      Tensor dx = empty_like_opts(sv[0].sizes(), sv[0]);
+      auto [dw, db] = conv_bwd(sv[0], sv[1], sv[2], dy, dx, sv[3]);
+      out = {dx, dw, db, Tensor()};
+    }
+    return once_differentiable(std::move(out), g, "the causal conv");
   }
 };
 
@@ -590,6 +621,10 @@ struct NormFn : Function<NormFn> {
     return {y};
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return once_differentiable(grads(ctx, g), g, "the LayerNorm");
+  }
+  static variable_list grads(AutogradContext* ctx, const variable_list& g) {
+    at::NoGradGuard no_grad;
     const auto sv = ctx->get_saved_variables();
     const Tensor &x2 = sv[0], &w = sv[1];
     const int64_t R = x2.size(0), E = x2.size(1);
@@ -701,7 +736,7 @@ struct InProjFn : Function<InProjFn> {
     const int64_t M = h2.size(0);
     Tensor out = empty_like_opts({M, O}, h);
     gemm(h2, W, out, gemm_desc(M, O, E, E, E, O, true, true));
-    ctx->save_for_backward({h2, W});
+    ctx->save_for_backward({h, W});
     auto shape = h.sizes().vec();
     ctx->saved_data["shape"] = shape;
     shape.back() = O;
@@ -709,10 +744,17 @@ struct InProjFn : Function<InProjFn> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto sv = ctx->get_saved_variables();
-    const Tensor &h2 = sv[0], &W = sv[1];
-    const int64_t O = W.size(0), E = W.size(1), M = h2.size(0);
-    const Tensor g2 = dense(g[0].reshape({M, O}));
+    const Tensor& W = sv[1];
+    const int64_t O = W.size(0), E = W.size(1);
     Tensor dh, dW;
+    if (at::GradMode::is_enabled()) {  // create_graph: products that have a derivative themselves
+      if (ctx->needs_input_grad(0)) dh = at::matmul(g[0], W);
+      if (ctx->needs_input_grad(1)) dW = at::matmul(g[0].reshape({-1, O}).t(), sv[0].reshape({-1, E}));
+      return {dh, dW};
+    }
+    const Tensor h2 = dense(sv[0].reshape({-1, E}));
+    const int64_t M = h2.size(0);
+    const Tensor g2 = dense(g[0].reshape({M, O}));
     if (ctx->needs_input_grad(0)) {
       dh = empty_like_opts({M, E}, g2);
       gemm(g2, W, dh, gemm_desc(M, E, O, O, E, E, true, false));
@@ -742,7 +784,7 @@ struct OutProjFn : Function<OutProjFn> {
       d.b_seg_stride = E * D;
     }
     gemm(y2, W, out, d, res.has_value() ? res->reshape({M, E}).contiguous() : Tensor());
-    ctx->save_for_backward({y2, W});
+    ctx->save_for_backward({y, W});
     ctx->saved_data["res"] = res.has_value();
     ctx->saved_data["shape"] = y.sizes().vec();
     auto shape = y.sizes().vec();
@@ -752,10 +794,20 @@ struct OutProjFn : Function<OutProjFn> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto sv = ctx->get_saved_variables();
-    const Tensor &y2 = sv[0], &W = sv[1];
-    const int64_t K = W.size(0), E = W.size(1), D = W.size(2), M = y2.size(0);
-    const Tensor g2 = dense(g[0].reshape({M, E}));
+    const Tensor& W = sv[1];
+    const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
     Tensor dy, dW;
+    const Tensor dres = ctx->saved_data["res"].toBool() ? g[0] : Tensor();
+    if (at::GradMode::is_enabled()) {  // as in InProjFn
+      const Tensor Wc = W.permute({1, 0, 2}).reshape({E, K * D});
+      if (ctx->needs_input_grad(0)) dy = at::matmul(g[0], Wc).view(ctx->saved_data["shape"].toIntVector());
+      if (ctx->needs_input_grad(1))
+        dW = at::matmul(g[0].reshape({-1, E}).t(), sv[0].reshape({-1, K * D})).view({E, K, D}).permute({1, 0, 2});
+      return {dy, dW, dres};
+    }
+    const Tensor y2 = dense(sv[0].reshape({-1, K * D}));
+    const int64_t M = y2.size(0);
+    const Tensor g2 = dense(g[0].reshape({M, E}));
     if (ctx->needs_input_grad(0)) {
       dy = empty_like_opts({M, K, D}, g2);
       auto d = gemm_desc(M, D, E, E, D, K * D, true, false);
@@ -773,7 +825,7 @@ struct OutProjFn : Function<OutProjFn> {
       d.c_stride_batch = E * D;
       gemm(g2, y2, dW, d);
     }
-    return {dy, dW, ctx->saved_data["res"].toBool() ? g[0] : Tensor()};
+    return {dy, dW, dres};
   }
 };
 
@@ -912,8 +964,16 @@ struct CoreFn : Function<CoreFn> {
     }
     return o.y;
   }
-  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return once_differentiable(grads(ctx, g), g, "the Mamba block's core");
+  }
+  static variable_list grads(AutogradContext* ctx, const variable_list& grads) {
     const auto sv = ctx->get_saved_variables();
+    // refused at once, except where dt_proj is frozen: there the first
+    // derivative was always given, and once_differentiable refuses the second
+    TORCH_CHECK(!(at::GradMode::is_enabled() && sv[4].requires_grad()),
+                "the Mamba block's core is not twice differentiable (create_graph=True)");
+    at::NoGradGuard no_grad;
     const Tensor &xz = sv[0], &conv_w = sv[1], &conv_b = sv[2], &W_x = sv[3], &W_dt = sv[4], &b_dt = sv[5],
                  &A_log = sv[6], &Dv = sv[7], &tok = sv[8], &xc = sv[9], &dbc = sv[10], &delta_raw = sv[11];
     const int64_t bsz = xz.size(0), n = xz.size(1), K = xz.size(2), din = xz.size(3) / 2;

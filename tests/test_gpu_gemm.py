@@ -182,3 +182,25 @@ def test_batched_matches_float64(cuda, q, m, k, n):
                     r2, S2 = ref + keep[..., :n].double(), S + keep[..., :n].double().abs()
                     assert ((out[..., :n].double() - r2).abs() <= bound * S2).all()
                     assert torch.equal(out[..., n:], keep[..., n:])
+
+
+def test_projections_are_twice_differentiable(cuda):
+    """Second derivatives of in_proj and out_proj against float64 autograd."""
+    gen = torch.Generator().manual_seed(1)
+    B, n, K, D, E = 2, 9, 2, 16, 12
+    h = torch.randn(B, n, E, generator=gen).cuda().requires_grad_()
+    Wi = torch.randn(K * D, E, generator=gen).cuda().requires_grad_()
+    Wo = torch.randn(K, E, D, generator=gen).cuda().requires_grad_()
+    res = torch.randn(B, n, E, generator=gen).cuda()
+
+    def second(out, ts):
+        gs = torch.autograd.grad(out.tanh().sum(), ts, create_graph=True)
+        return torch.autograd.grad(sum(g.square().sum() for g in gs), ts)
+
+    got = second(gemm.out_proj(gemm.in_proj(h, Wi).view(B, n, K, D), Wo) + res, (h, Wi, Wo))
+    hd, wi, wo = [t.detach().double().cpu().requires_grad_() for t in (h, Wi, Wo)]
+    out = torch.einsum("bnkd,ked->bne", (hd @ wi.t()).view(B, n, K, D), wo) + res.double().cpu()
+    for a, r in zip(got, second(out, (hd, wi, wo))):
+        # tanh's argument is off by the products' roundings (a few 2^-24 of a sum of 100), its second
+        # derivative by as much again
+        assert (a.double().cpu() - r).norm() <= 1e-4 * r.norm()

@@ -11,7 +11,7 @@ import mlx_vision_mamba_amd as mvm
 from mlx_vision_mamba_amd import _lib, scan, synthetic
 from mlx_vision_mamba_amd.conv import causal_conv_silu
 from mlx_vision_mamba_amd.norm import layer_norm
-from oracle import ref_lib
+from oracle import ref_lib, torch_ref
 
 pytestmark = pytest.mark.gpu
 
@@ -219,3 +219,59 @@ def test_traced_modules_compute(cuda, make):
     with torch.no_grad():
         assert torch.equal(t(x), m(x))
         assert t(x).grad_fn is None
+
+
+@pytest.mark.parametrize("grid", [(4, 5), (37, 57)])  # 160 and 16,872 batch x rows
+def test_second_derivative_of_a_block_raises(cuda, grid):
+    """The core's backward is raw launches: asked for a graph of it, the block
+    refuses (with frozen parameters, where the first derivative was always
+    given, as soon as a derivative through it is taken)."""
+    torch.manual_seed(0)
+    m = mvm.MultiDirectionalMambaBlock(32, d_state=4, num_directions=4, grid_shape=grid, scan_mode="hip").to(cuda)
+    x = torch.randn(2, grid[0] * grid[1], 32, generator=torch.Generator().manual_seed(1)).to(cuda).requires_grad_()
+    ref = torch.autograd.grad(m(x).square().sum(), x)[0]
+    with pytest.raises(RuntimeError, match="not twice differentiable"):
+        torch.autograd.grad(m(x).square().sum(), x, create_graph=True)
+    m.requires_grad_(False)
+    (g,) = torch.autograd.grad(m(x).square().sum(), x, create_graph=True)
+    assert torch.allclose(g, ref, rtol=1e-4, atol=1e-4 * ref.abs().max().item())
+    with pytest.raises(RuntimeError, match="not twice differentiable"):
+        torch.autograd.grad(g.square().sum(), x)
+    with pytest.raises(RuntimeError, match="not twice differentiable"):
+        (m(x).sum() + g.square().sum()).backward()
+
+
+@pytest.mark.parametrize("make", [_Norm, _Conv, _Scan], ids=["norm", "conv", "scan"])
+def test_second_derivative_of_the_kernels_raises(cuda, make):
+    """create_graph gives the same first derivatives; a derivative through
+    them raises instead of lacking the kernel's part."""
+    m = make().to(cuda)
+    x = torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(1)).to(cuda).requires_grad_()
+    ps = [x, *m.parameters()]
+    ref = torch.autograd.grad(m(x).square().sum(), ps)
+    got = torch.autograd.grad(m(x).square().sum(), ps, create_graph=True)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+    for p in (x, ps[-1]):
+        with pytest.raises(RuntimeError, match="not twice differentiable"):
+            torch.autograd.grad(sum(a.square().sum() for a in got), p, retain_graph=True)
+
+
+def test_gradient_of_out_proj_is_differentiable(cuda):
+    """A penalty on the gradient of out_proj's weight: its graph leads through
+    the core's first derivative only.  Against the float64 restatement."""
+    torch.manual_seed(0)
+    m = mvm.MambaBlock(32, d_state=4, scan_mode="hip").to(cuda)
+    x = torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(1))
+
+    def penalty(y, w, xx):
+        (g,) = torch.autograd.grad(y.square().sum(), w, create_graph=True)
+        return torch.autograd.grad(g.square().sum(), [xx, w])
+
+    xg = x.to(cuda).requires_grad_()
+    got = penalty(m(xg), m.out_proj.weight, xg)
+    params = torch_ref.params_from_module(m)
+    xd = x.double().requires_grad_()
+    ref = penalty(torch_ref.mamba_block(params, "", xd, d_state=4, d_conv=4), params["out_proj.weight"], xd)
+    for a, r in zip(got, ref):
+        assert (a.double().cpu() - r).norm() <= 1e-5 * r.norm()
