@@ -254,12 +254,16 @@ at::ScalarType out_type(std::optional<at::ScalarType> dt, at::ScalarType in_dt) 
   return t;
 }
 
+// (y, checkpoints); y is (B, L, D) when flat.  It is allocated in that shape:
+// a view made inside a Function could not be changed in place
 std::pair<Tensor, Tensor> scan_fwd(const ScanIn& s, const Tensor& tok, int64_t chunk_len,
-                                   std::optional<at::ScalarType> out_dtype, bool save_ckpt) {
+                                   std::optional<at::ScalarType> out_dtype, bool save_ckpt, bool flat) {
   const auto out_dt = out_type(out_dtype, s.in_dt);
   const auto d = make_desc(s.u, s.Bm, s.in_dt, out_dt, tok, chunk_len);
   c10::OptionalDeviceGuard guard(s.u.device());
-  Tensor y = empty_like_opts(s.u.sizes(), s.u, out_dt), ckpt;
+  Tensor y = flat ? empty_like_opts({s.u.size(0), s.u.size(1), s.u.size(3)}, s.u, out_dt)
+                  : empty_like_opts(s.u.sizes(), s.u, out_dt);
+  Tensor ckpt;
   if (save_ckpt) ckpt = empty_like_opts({check(mvm_scan_ckpt_elems(&d))}, s.u);
   const int64_t nbytes = check(mvm_scan_workspace_bytes(&d, 0));
   const Tensor ws = workspace(nbytes, s.u);
@@ -315,12 +319,13 @@ struct ScanFn : Function<ScanFn> {
                         int64_t chunk_len, std::optional<at::ScalarType> out_dtype, bool needs, bool flat) {
     const Tensor tok = tok_.value_or(Tensor());
     const auto t = lift({u, delta, A, Bm, Cm, Dv}, flat);
-    auto [y, ckpt] = scan_fwd(prepare(t[0], t[1], t[2], t[3], t[4], t[5]), tok, chunk_len, out_dtype, needs);
+    auto [y, ckpt] = scan_fwd(prepare(t[0], t[1], t[2], t[3], t[4], t[5]), tok, chunk_len, out_dtype, needs,
+                              flat);
     ctx->saved_data["chunk"] = chunk_len;
     ctx->saved_data["out"] = out_dtype.has_value() ? static_cast<int64_t>(*out_dtype) : int64_t{-1};
     ctx->saved_data["flat"] = flat;
     if (needs) ctx->save_for_backward({u, delta, A, Bm, Cm, Dv, ckpt, tok});
-    return flat ? y.squeeze(2) : y;
+    return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto sv = ctx->get_saved_variables();
@@ -362,8 +367,8 @@ std::pair<Tensor, OptTensor> scan_forward(const Tensor& u, const Tensor& delta, 
   return guarded([&]() -> std::pair<Tensor, OptTensor> {
     const auto t = lift({u, delta, A, Bm, Cm, Dv}, flat);
     auto [y, ckpt] = scan_fwd(prepare(t[0], t[1], t[2], t[3], t[4], t[5]), tok.value_or(Tensor()), chunk_len,
-                              out_dtype, save_ckpt);
-    return {flat ? y.squeeze(2) : y, ckpt.defined() ? OptTensor(ckpt) : std::nullopt};
+                              out_dtype, save_ckpt, flat);
+    return {y, ckpt.defined() ? OptTensor(ckpt) : std::nullopt};
   });
 }
 
@@ -734,13 +739,13 @@ struct InProjFn : Function<InProjFn> {
     const int64_t O = W.size(0), E = W.size(1);
     const Tensor h2 = dense(h.reshape({-1, E}));
     const int64_t M = h2.size(0);
-    Tensor out = empty_like_opts({M, O}, h);
-    gemm(h2, W, out, gemm_desc(M, O, E, E, E, O, true, true));
-    ctx->save_for_backward({h, W});
     auto shape = h.sizes().vec();
     ctx->saved_data["shape"] = shape;
     shape.back() = O;
-    return out.view(shape);
+    Tensor out = empty_like_opts(shape, h);  // (not a view: see OutProjFn)
+    gemm(h2, W, out, gemm_desc(M, O, E, E, E, O, true, true));
+    ctx->save_for_backward({h, W});
+    return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto sv = ctx->get_saved_variables();
@@ -777,7 +782,12 @@ struct OutProjFn : Function<OutProjFn> {
     const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
     const Tensor y2 = dense(y.reshape({-1, K * D}));
     const int64_t M = y2.size(0);
-    Tensor out = empty_like_opts({M, E}, y);
+    // allocated in its final shape: a view made here could not be changed in place
+    auto shape = y.sizes().vec();
+    ctx->saved_data["shape"] = shape;
+    shape.pop_back();
+    shape.back() = E;
+    Tensor out = empty_like_opts(shape, y);
     auto d = gemm_desc(M, E, K * D, K * D, D, E, true, true);
     if (K > 1) {
       d.b_seg = D;
@@ -786,11 +796,7 @@ struct OutProjFn : Function<OutProjFn> {
     gemm(y2, W, out, d, res.has_value() ? res->reshape({M, E}).contiguous() : Tensor());
     ctx->save_for_backward({y, W});
     ctx->saved_data["res"] = res.has_value();
-    ctx->saved_data["shape"] = y.sizes().vec();
-    auto shape = y.sizes().vec();
-    shape.pop_back();
-    shape.back() = E;
-    return out.view(shape);
+    return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto sv = ctx->get_saved_variables();

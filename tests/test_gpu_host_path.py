@@ -275,3 +275,27 @@ def test_gradient_of_out_proj_is_differentiable(cuda):
     ref = penalty(torch_ref.mamba_block(params, "", xd, d_state=4, d_conv=4), params["out_proj.weight"], xd)
     for a, r in zip(got, ref):
         assert (a.double().cpu() - r).norm() <= 1e-5 * r.norm()
+
+
+@pytest.mark.parametrize("make", [
+    lambda: mvm.MambaBlock(32, d_state=4, scan_mode="hip"),
+    lambda: mvm.ResidualMambaBlock(32, d_state=4, scan_mode="hip"),
+    lambda: mvm.BidirectionalMambaBlock(32, d_state=4, scan_mode="hip"),
+    lambda: mvm.MultiDirectionalMambaBlock(32, d_state=4, num_directions=4, grid_shape=(4, 5), scan_mode="hip"),
+    _Conv, _Scan], ids=["mamba", "residual", "bidirectional", "multi", "conv", "scan"])
+def test_outputs_can_be_changed_in_place(cuda, make):
+    """No output is a view made inside a Function: in-place changes of it are
+    recorded as those of any other tensor."""
+    torch.manual_seed(0)
+    m = make().to(cuda)
+    x = torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(1)).to(cuda).requires_grad_()
+    w = torch.randn(32, generator=torch.Generator().manual_seed(2)).to(cuda).requires_grad_()
+    ps = [x, w, *m.parameters()]
+    y = m(x)
+    ref = torch.autograd.grad(torch.relu((y + w) * 2).square().sum(), ps)
+    y = m(x)
+    y += w
+    y.mul_(2)
+    torch.relu_(y)
+    for a, b in zip(torch.autograd.grad(y.square().sum(), ps), ref):
+        assert torch.equal(a, b)
