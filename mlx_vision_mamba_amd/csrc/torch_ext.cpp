@@ -55,6 +55,15 @@ std::string shape_str(const Tensor& t) {
   return s + (t.dim() == 1 ? ",)" : ")");
 }
 
+// sets the Python error that stands for e (with the GIL held)
+void set_scan_error(const StatusError& e) {
+  const std::string msg = e.what();
+  const py::object cls = py::module_::import("mlx_vision_mamba_amd._lib").attr("ScanError");
+  const auto cut = msg.find(": ");
+  const py::object exc = cls(e.code, msg.substr(cut == std::string::npos ? 0 : cut + 2));
+  PyErr_SetObject(cls.ptr(), exc.ptr());
+}
+
 // Runs f with torch's exception translation, and StatusError as ScanError
 template <typename F>
 auto guarded(F&& f) -> decltype(f()) {
@@ -62,14 +71,30 @@ auto guarded(F&& f) -> decltype(f()) {
   try {
     return f();
   } catch (const StatusError& e) {
-    const std::string msg = e.what();
-    py::object cls = py::module_::import("mlx_vision_mamba_amd._lib").attr("ScanError");
-    const auto cut = msg.find(": ");
-    py::object exc = cls(e.code, msg.substr(cut == std::string::npos ? 0 : cut + 2));
-    PyErr_SetObject(cls.ptr(), exc.ptr());
+    set_scan_error(e);
     throw py::error_already_set();
   }
   END_HANDLE_TH_ERRORS_PYBIND
+}
+
+// Runs a Function's backward: the autograd engine carries its exceptions from
+// its own threads to the caller's, but hands a C++ one over as RuntimeError.
+// Library refusals and ValueErrors travel as the Python exceptions they are.
+template <typename F>
+variable_list in_backward(F&& f) {
+  python_error err;
+  try {
+    return f();
+  } catch (const StatusError& e) {
+    py::gil_scoped_acquire gil;
+    set_scan_error(e);
+    err.persist();
+  } catch (const py::builtin_exception& e) {
+    py::gil_scoped_acquire gil;
+    e.set_error();
+    err.persist();
+  }
+  throw python_error(std::move(err));
 }
 
 // ---------------------------------------------------------------- helpers
@@ -328,6 +353,9 @@ struct ScanFn : Function<ScanFn> {
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return in_backward([&] { return grads(ctx, g); });
+  }
+  static variable_list grads(AutogradContext* ctx, const variable_list& g) {
     const auto sv = ctx->get_saved_variables();
     const bool flat = ctx->saved_data["flat"].toBool();
     const int64_t od = ctx->saved_data["out"].toInt();
@@ -581,6 +609,9 @@ struct ConvFn : Function<ConvFn> {
     return y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return in_backward([&] { return grads(ctx, g); });
+  }
+  static variable_list grads(AutogradContext* ctx, const variable_list& g) {
     const auto sv = ctx->get_saved_variables();
     variable_list out;
     {
@@ -626,7 +657,7 @@ struct NormFn : Function<NormFn> {
     return {y};
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
-    return once_differentiable(grads(ctx, g), g, "the LayerNorm");
+    return in_backward([&] { return once_differentiable(grads(ctx, g), g, "the LayerNorm"); });
   }
   static variable_list grads(AutogradContext* ctx, const variable_list& g) {
     at::NoGradGuard no_grad;
@@ -748,6 +779,9 @@ struct InProjFn : Function<InProjFn> {
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return in_backward([&] { return grads(ctx, g); });
+  }
+  static variable_list grads(AutogradContext* ctx, const variable_list& g) {
     const auto sv = ctx->get_saved_variables();
     const Tensor& W = sv[1];
     const int64_t O = W.size(0), E = W.size(1);
@@ -799,6 +833,9 @@ struct OutProjFn : Function<OutProjFn> {
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
+    return in_backward([&] { return grads(ctx, g); });
+  }
+  static variable_list grads(AutogradContext* ctx, const variable_list& g) {
     const auto sv = ctx->get_saved_variables();
     const Tensor& W = sv[1];
     const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
@@ -971,7 +1008,7 @@ struct CoreFn : Function<CoreFn> {
     return o.y;
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
-    return once_differentiable(grads(ctx, g), g, "the Mamba block's core");
+    return in_backward([&] { return once_differentiable(grads(ctx, g), g, "the Mamba block's core"); });
   }
   static variable_list grads(AutogradContext* ctx, const variable_list& grads) {
     const auto sv = ctx->get_saved_variables();

@@ -299,3 +299,21 @@ def test_outputs_can_be_changed_in_place(cuda, make):
     torch.relu_(y)
     for a, b in zip(torch.autograd.grad(y.square().sum(), ps), ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which,change,error,match", [
+    ("u", lambda t: t[:, :-1], ValueError, "equal shape"),
+    ("ckpt", lambda t: torch.cat([t[:1], t])[1:], _lib.ScanError, "16-byte aligned"),
+    ("u", lambda t: t.cpu(), RuntimeError, "only on the GPU")])
+def test_error_types_of_a_backward(cuda, which, change, error, match):
+    """What a backward's host checks refuse (here: saved tensors that a hook
+    hands back changed) keeps its type through the autograd engine."""
+    u, *ins = [t.to(cuda) for t in synthetic.make(1, 20, 8, 4, seed=0)[:6]]
+    pick = {"u": lambda t: t.shape == u.shape and torch.equal(t, u), "ckpt": lambda t: t.dim() == 1 and t.numel() > 8}
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: change(t) if pick[which](t) else t):
+        y = scan.selective_scan(u.clone().requires_grad_(), *ins)
+    with pytest.raises(error, match=match) as e:
+        y.sum().backward()
+    assert type(e.value) is error
+    if error is _lib.ScanError:
+        assert e.value.code == _lib.MVM_ERR_INVALID_ARG
