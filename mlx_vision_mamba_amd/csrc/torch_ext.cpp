@@ -717,9 +717,10 @@ constexpr int64_t kMaxLd = int64_t{1} << 21;
 constexpr int64_t kStreamRows = 16384;
 
 // out[q] (+)= op(A[q]) @ op(B[q]) for float32 (batch, rows, cols) views; ta /
-// tb transpose an operand.  The kernels take contiguous columns, and 16-byte
-// rows of an operand whose summed index is the contiguous one (from 32 summed
-// values up); other operands, and `stream` products of many rows, are torch's.
+// tb transpose an operand.  The kernels take contiguous columns, operand rows
+// that do not overlap, and 16-byte rows of an operand whose summed index is the
+// contiguous one (from 32 summed values up); other operands (a parameter that
+// is an expanded row, say), and `stream` products of many rows, are torch's.
 void batched(const Tensor& A, const Tensor& B, Tensor& out, bool ta, bool tb, bool accumulate, bool stream) {
   TORCH_CHECK(A.dim() == 3 && B.dim() == 3 && out.dim() == 3, "batched products take 3-D tensors");
   const int64_t q = A.size(0), m = A.size(ta ? 2 : 1), k = A.size(ta ? 1 : 2), n = B.size(tb ? 1 : 2);
@@ -730,8 +731,8 @@ void batched(const Tensor& A, const Tensor& B, Tensor& out, bool ta, bool tb, bo
   for (const Tensor* t : {&A, &B, static_cast<const Tensor*>(&out)})
     TORCH_CHECK(t->scalar_type() == at::kFloat, "batched products take float32; got ", t->scalar_type());
   auto rows16 = [](const Tensor& t) { return t.stride(1) % 4 == 0 && t.stride(0) % 4 == 0 && aligned16(t); };
-  const bool ok = A.stride(2) == 1 && B.stride(2) == 1 && out.stride(2) == 1 && A.stride(1) < kMaxLd &&
-                  B.stride(1) < kMaxLd && (k < 32 || ((ta || rows16(A)) && (!tb || rows16(B)))) &&
+  auto rows = [](const Tensor& t) { return t.stride(2) == 1 && t.stride(1) >= t.size(2) && t.stride(1) < kMaxLd; };
+  const bool ok = rows(A) && rows(B) && out.stride(2) == 1 && (k < 32 || ((ta || rows16(A)) && (!tb || rows16(B)))) &&
                   !(stream && q * m > kStreamRows);
   if (ok) {
     auto d = gemm_desc(m, n, k, A.stride(1), B.stride(1), out.stride(1), !ta, tb);

@@ -204,3 +204,36 @@ def test_projections_are_twice_differentiable(cuda):
         # tanh's argument is off by the products' roundings (a few 2^-24 of a sum of 100), its second
         # derivative by as much again
         assert (a.double().cpu() - r).norm() <= 1e-4 * r.norm()
+
+
+@pytest.mark.parametrize("tb", [False, True])
+def test_batched_takes_overlapping_and_single_rows(cuda, tb):
+    """Operands with rows that share memory (an expanded row), or one row of
+    any stride: torch's product, as for other layouts the kernels do not take."""
+    gen = torch.Generator().manual_seed(1)
+    rn = lambda *s: torch.randn(*s, generator=gen).cuda()  # noqa: E731
+    a = rn(2, 37, 40)
+    b = (rn(2, 1, 40).expand(2, 24, 40) if tb else rn(2, 1, 24).expand(2, 40, 24))
+    one = rn(2 * 40).as_strided((2, 1, 40), (40, 1, 1))
+    for A in (a, one):
+        ref = A.double() @ (b.transpose(1, 2) if tb else b).contiguous().double()
+        S = A.double().abs() @ (b.transpose(1, 2) if tb else b).contiguous().double().abs()
+        # (any order of 40 float32 additions)
+        assert ((gemm.batched(A, b, tb=tb).double() - ref).abs() <= 42 * 2.0 ** -24 * S).all()
+
+
+def test_block_with_an_expanded_projection(cuda):
+    """x_proj's weight as one row for all outputs: the block of the same values
+    laid out in full."""
+    import mlx_vision_mamba_amd as mvm
+    torch.manual_seed(0)
+    m = mvm.MambaBlock(32, d_state=4, scan_mode="hip").to(cuda)
+    x = torch.randn(2, 20, 32, generator=torch.Generator().manual_seed(1)).to(cuda)
+    w = m.x_proj.weight.detach()[:1].expand(m.x_proj.weight.shape)
+    out = []
+    for v in (w, w.clone()):
+        m.x_proj.weight = torch.nn.Parameter(v)
+        y = m(x)
+        out.append([y, *torch.autograd.grad(y.sum(), m.parameters())])
+    for p, q in zip(*out):
+        assert (p - q).abs().max() <= 1e-5 * q.abs().max()
