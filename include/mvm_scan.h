@@ -119,6 +119,13 @@ int64_t mvm_scan_workspace_bytes(const mvm_scan_desc* desc, int which);
  * without checkpoints and with bf16 results may take longer chunks). */
 int64_t mvm_scan_chunk_len(const mvm_scan_desc* desc);
 
+/* A time-chunk length that can be longer than that, and faster (a forward and
+ * VJP of 3 x 1037 positions of 1000 channels: 103 us instead of 111), for a
+ * caller whose results round more than the scan: against float64 dA is off by
+ * up to 3.1e-7 instead of 2.3e-7.  Pass it as chunk_len, to the forward and to
+ * the VJP.  (chunk_len > 0 in `desc` is returned as it is.) */
+int64_t mvm_scan_long_chunk_len(const mvm_scan_desc* desc);
+
 /* Forward scan.  y may be NULL (checkpoints only); ckpt may be NULL
  * (inference).  delta is float32.  See the header comment for layouts. */
 int mvm_scan_fwd(const mvm_scan_desc* desc, const void* u, const float* delta,
@@ -205,9 +212,6 @@ int mvm_scan_fused_validate(const mvm_scan_fused_desc* desc);
  * (which = 1); gate != 0 when z is given.  Checkpoints are sized by
  * mvm_scan_ckpt_elems(&desc->scan). */
 int64_t mvm_scan_fused_workspace_bytes(const mvm_scan_fused_desc* desc, int which, int gate);
-
-/* Time-chunk length the fused scans will use for this descriptor. */
-int64_t mvm_scan_fused_chunk_len(const mvm_scan_fused_desc* desc);
 
 /* y = scan(u, softplus(delta_raw + delta_bias), A, Bm, Cm, Dv) * silu(z).
  * delta_bias (ndir, dim) may be NULL (zero bias); z may be NULL (no gate,

@@ -69,9 +69,9 @@ constexpr int64_t kMaxSeqlen = INT32_MAX - 64;
 // bits dA is off by 2.3e-7 at 32 positions, 3.1e-7 at 64 and 4.1e-7 unchunked
 // (B=16 L=512 D=768), y by 3.3e-8, 3.5e-8 and 3.6e-8.  So `longer` is for calls
 // whose results do not show it: bf16 forwards without checkpoints (their
-// rounding is 1.7e-3) and the fused scan, where the block's products decide
-// (all gradients of blocks of L=331 and 512 are off by 2-4.6e-7, A_log's by
-// 3.0-3.6e-7).
+// rounding is 1.7e-3) and callers that ask for it (mvm_scan_long_chunk_len): a
+// block, where its products decide (all gradients of blocks of L=331 and 512
+// are off by 2-4.6e-7, A_log's by 3.0-3.6e-7).
 int64_t pick_chunk_len(const mvm_scan_desc* d, bool longer) {
   if (d->chunk_len > 0) return d->chunk_len;
   const int64_t tiles = ceil_div(d->seqlen, mvm::kSub);
@@ -258,6 +258,12 @@ int64_t mvm_scan_chunk_len(const mvm_scan_desc* desc) {
   const int rc = check_desc(desc);
   if (rc != MVM_OK) return rc;
   return make_geom(desc).chunk_len;
+}
+
+int64_t mvm_scan_long_chunk_len(const mvm_scan_desc* desc) {
+  const int rc = check_desc(desc);
+  if (rc != MVM_OK) return rc;
+  return pick_chunk_len(desc, true);
 }
 
 int mvm_scan_fwd(const mvm_scan_desc* desc, const void* u, const float* delta, const float* A,
@@ -473,7 +479,7 @@ bool z_ok(const mvm_scan_fused_desc* fd) {
 }
 
 mvm::Geom fused_geom(const mvm_scan_fused_desc* fd) {
-  mvm::Geom g = make_geom(&fd->scan, true);
+  mvm::Geom g = make_geom(&fd->scan);
   g.dsb = fd->dt_stride_b; g.dsk = fd->dt_stride_k; g.dst = fd->dt_stride_t;
   g.ysb = fd->y_stride_b;  g.ysk = fd->y_stride_k;  g.yst = fd->y_stride_t;
   g.zsb = fd->z_stride_b;  g.zsk = fd->z_stride_k;  g.zst = fd->z_stride_t;
@@ -510,12 +516,6 @@ extern "C" {
 int mvm_scan_fused_validate(const mvm_scan_fused_desc* desc) {
   const int rc = check_fused(desc);
   return rc == MVM_OK ? ok() : rc;
-}
-
-int64_t mvm_scan_fused_chunk_len(const mvm_scan_fused_desc* desc) {
-  const int rc = check_fused(desc);
-  if (rc != MVM_OK) return rc;
-  return fused_geom(desc).chunk_len;
 }
 
 int64_t mvm_scan_fused_workspace_bytes(const mvm_scan_fused_desc* desc, int which, int gate) {

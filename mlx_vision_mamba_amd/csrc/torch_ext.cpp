@@ -998,6 +998,11 @@ struct CoreFn : Function<CoreFn> {
     // (forward only: delta_raw is never formed in memory; xc lends its layout)
     Tensor delta_raw = dt_in && !save ? xc : empty_like_opts({K, M, din}, xz);
     if (!dt_in) batched(dbc.narrow(2, 0, R), W_dt, delta_raw, false, true, false, true);
+    // (the products of a block round more than its scan does)
+    if (chunk_len == 0) {
+      const auto d = make_desc(bnkd(xc, bsz, n), bc.narrow(3, R, ns), at::kFloat, at::kFloat, tok, 0);
+      chunk_len = check(mvm_scan_long_chunk_len(&d));
+    }
     const auto o = fused_fwd(bnkd(xc, bsz, n), bnkd(delta_raw, bsz, n), b_dt, A_log, bc.narrow(3, R, ns),
                              bc.narrow(3, R + ns, ns), Dv, z, tok, chunk_len, save, true,
                              dt_in ? bc.narrow(3, 0, R) : Tensor(), W_dt);                  // :180-190

@@ -321,18 +321,14 @@ def get_scan_fn(scan_mode: str):
 def chunk_len_for(rows, L, D, N=16, fused=False):
     """Time-chunk length the library picks for `rows` = batch x directions
     scans of length L over D channels (the whole sequence when it is one
-    chunk); ``fused``: for the fused scans of the blocks."""
+    chunk); ``fused``: the one that the blocks pass to their fused scans."""
     d = _lib.ScanDesc()
     d.batch, d.seqlen, d.dim, d.dstate, d.ndir = rows, L, D, N, 1
     d.x_stride_b, d.x_stride_k, d.x_stride_t = L * D, 0, D
     d.bc_stride_b, d.bc_stride_k, d.bc_stride_t = L * N, 0, N
     d.in_dtype = d.out_dtype = _lib.MVM_F32
     if fused:
-        f = _lib.FusedDesc()
-        f.scan = d
-        f.dt_stride_b, f.dt_stride_k, f.dt_stride_t = L * D, 0, D
-        f.y_stride_b, f.y_stride_k, f.y_stride_t = L * D, 0, D
-        return _lib.check(_lib.lib().mvm_scan_fused_chunk_len(ctypes.byref(f)))
+        return _lib.check(_lib.lib().mvm_scan_long_chunk_len(ctypes.byref(d)))
     return _lib.check(_lib.lib().mvm_scan_chunk_len(ctypes.byref(d)))
 
 

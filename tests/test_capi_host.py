@@ -482,3 +482,26 @@ def test_dt_columns_stay_inside_the_row():
         assert n >= rank and got[:rank] == list(range(rank))
         assert max(got) < rank, rank
     assert _lib.lib().mvm_selftest_dt_columns(49, cols) == _lib.MVM_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("B,L,D", [(16, 512, 768), (3, 1037, 1000), (10, 331, 400), (1, 4096, 768), (32, 196, 3072)])
+def test_fused_scans_take_the_default_chunks(B, L, D):
+    """A fused scan that is given no chunk length takes the plain scan's (the
+    shorter ones, which round less), as its workspace shows; the longer ones
+    are the caller's choice."""
+    d = _desc(B=B, L=L, D=D)
+    f = _lib.FusedDesc()
+    f.scan = d
+    for k in ("dt", "y", "z"):
+        for ax, v in (("b", L * D), ("t", D), ("k", D)):
+            setattr(f, f"{k}_stride_{ax}", v)
+    lib = _lib.lib()
+    for which in (0, 1):
+        need = _lib.check(lib.mvm_scan_fused_workspace_bytes(ctypes.byref(f), which, 1))
+        f.scan.chunk_len = _lib.check(lib.mvm_scan_chunk_len(ctypes.byref(d)))
+        assert _lib.check(lib.mvm_scan_fused_workspace_bytes(ctypes.byref(f), which, 1)) == need
+        f.scan.chunk_len = 0
+    longer = _lib.check(lib.mvm_scan_long_chunk_len(ctypes.byref(d)))
+    assert longer % 16 == 0 and longer >= lib.mvm_scan_chunk_len(ctypes.byref(d))
+    d.chunk_len = 48
+    assert lib.mvm_scan_long_chunk_len(ctypes.byref(d)) == 48
