@@ -23,8 +23,10 @@
  * matrix of its own, in one product over K * d_inner).
  *
  * The products run on the bf16 matrix units with every float32 operand split
- * exactly into three bf16 parts; see csrc/gemm.hip for the error.  Results
- * are bitwise deterministic.  Conventions are those of mvm_scan.h (status
+ * exactly into three bf16 parts; see csrc/gemm.hip for the error.  Where the
+ * split cannot hold the values (infinities, NaN, results to which values below
+ * 2^-110 matter) the float32 units compute the tile's part again: the results
+ * are float32's, but up to five times slower.  Results are bitwise deterministic.  Conventions are those of mvm_scan.h (status
  * codes, mvm_last_error, caller-owned buffers, host-side validation before
  * any launch, no device allocation).  C must not overlap A or B.
  */

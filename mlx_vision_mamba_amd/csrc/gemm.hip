@@ -22,12 +22,29 @@
 // against float64 1.1e-7 at k = 384 and 2.7e-7 at k = 6144 in 3 parts (normal
 // inputs; the BLAS library's float32 matrix instructions: 3.5e-7 and 1.4e-6).
 //
-// What the split cannot hold, and what is done: infinities and NaN (and
+// What the split cannot hold, and what is done.  Infinities and NaN (and
 // values above the largest bf16, which round to infinity) make a NaN out of
-// hi - hi, and below 2^-109 the low parts underflow.  A wave whose results
-// are not all finite, or all so small (below 2^-64, not all zero) that their
-// inputs may have been, computes its part of the tile again with the float32
-// matrix instructions, which have neither limit.
+// hi - hi.  Below 2^-110 the low parts are finer than bf16's smallest subnormal
+// and lose up to 2^-134, which a result c shows only if it is small beside the
+// other operand: len 2^-133 max(|A|, |B|) > 2^-24 |c|.  And products of parts
+// below 2^-126 may be lost, which shows in |c| < 6 len 2^-102.  So every thread
+// keeps the largest magnitude of its share of the row (or column) it stages,
+// one instruction per two values, and a wave computes its part of the tile
+// again with the float32 matrix instructions, which have none of these limits,
+// when
+//   - a result is not finite;
+//   - a row or a column it uses is nonzero but below 2^-110 throughout (its
+//     results may have lost everything); or
+//   - a nonzero result is below one of the two bounds.
+// Rows and columns are looked at, through LDS, only in a tile with a thread
+// whose share is tiny or holds a value from 2^10 up; elsewhere the second bound
+// is the higher one.  (Left out: a result of exactly zero to which, in a row and
+// a column that hold normal values, only products with values below 2^-134
+// contribute.)  The bookkeeping costs 1-1.5 % (6272 x 6144 x 384: 182-187 us
+// without it, 184-188 with it).  The second computation reads its operands from
+// global memory value by value: there, 200 us become 385 with one NaN in A, 350
+// with A of order 2^-80 and 950 with an infinity in every row; the library's
+// float32 kernels stay at 265.
 //
 // Work split: a 256-thread workgroup computes a BM x BN tile, its 4 waves
 // (2 x 2) a quarter each in 32x32x16 MFMA tiles.  Both operands are split
@@ -63,10 +80,18 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kGroupM = 8;  // row tiles per group of the tile order
+constexpr float kLarge = 0x1p10f;  // up to here the second bound below is the higher one
 
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   const f32x2 v = {a, b};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// max(m, |a|, |b|), NaN if one of them is, in one instruction (from fmaxf or
+// the maximum builtins the compiler makes up to three)
+__device__ __forceinline__ float max3_abs(float m, float a, float b) {
+  asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
+  return m;
 }
 
 // the three bf16 planes of 8 values
@@ -144,9 +169,14 @@ struct Operand {
   __device__ static __forceinline__ int swz(int r, int c) {
     return BK == 16 ? (c ^ (((r >> 2) ^ (r >> 3)) & 1)) * 8 : (c ^ (((r >> 1) ^ (r >> 3)) & 3)) * 8;
   }
-  __device__ __forceinline__ void store(uint16_t (*lds)[ROWS][BK], const float (&v)[kItems][8]) const {
+  // (kItems is 1: the thread's values all belong to one row, whose largest
+  // magnitude it keeps in `top`)
+  static_assert(kItems == 1, "one row per thread");
+  __device__ __forceinline__ void store(uint16_t (*lds)[ROWS][BK], const float (&v)[kItems][8], float& top) const {
 #pragma unroll
     for (int i = 0; i < kItems; ++i) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) top = max3_abs(top, v[i][e], v[i][e + 1]);
       uint4 pl[3];
       split8(v[i], pl);
       const int o = swz(row[i], chunk[i]);
@@ -163,6 +193,8 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
   constexpr int MT = BM / 64, NT = BN / 64;  // 32 x 32 tiles of a wave
   __shared__ __attribute__((aligned(16))) uint16_t sA[2][3][BM][BK];
   __shared__ __attribute__((aligned(16))) uint16_t sB[2][3][BN][BK];
+  __shared__ uint32_t sTop[BM + BN];  // largest magnitude of each row of A and column of B, as bits
+  __shared__ __attribute__((aligned(16))) uint32_t sLook[kThreads / 64];  // a wave's reason to form them
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -217,9 +249,17 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
       }
     }
   };
+  float topa = 0.f, topb = 0.f;
   auto stage = [&](int buf, int r) {
-    oa.store(sA[buf], pa[r]);
-    ob.store(sB[buf], pb[r]);
+    oa.store(sA[buf], pa[r], topa);
+    ob.store(sB[buf], pb[r], topb);
+  };
+  // before the last barrier: whether a thread's share of a row or column is
+  // tiny throughout, or any value is large
+  auto tiny = [](float t) { return t > 0.f && t < 0x1p-110f; };
+  auto note = [&] {
+    const bool look = __ballot(tiny(topa) || tiny(topb) || fmaxf(topa, topb) >= kLarge) != 0;
+    if (lane == 0) sLook[wave] = look;
   };
 
   // hi * hi, and the five smaller products (added at the end)
@@ -272,6 +312,7 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
       __syncthreads();
       compute(0);
     }
+    note();
     __syncthreads();
   }
   if (len > full * BK) {  // (segments are whole steps: no segment ends in a partial one)
@@ -281,26 +322,53 @@ gemm_kernel(GemmGeom g, const float* __restrict__ A, const float* __restrict__ B
     oa.load_tail(pa[0], A0 + done * astep, g.lda, len - full * BK);
     ob.load_tail(pb[0], B0 + bo, g.ldb, len - full * BK);
     stage(0, 0);
+    note();
     __syncthreads();
     compute(0);
   }
 
   // results the split cannot vouch for: again with the float32 instructions
-  float big = 0.f;
-  bool finite = true;
+  float most = 0.f;               // the largest magnitude (NaN: one of them is)
+  uint32_t least = 0xffffffffu;  // the smallest that is not zero: 2 |bits| - 1
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NT; ++j) {
+      acc[i][j] += acs[i][j];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        acc[i][j][r] += acs[i][j][r];
-        const float x = fabsf(acc[i][j][r]);
-        finite &= x < __builtin_inff();
-        big = fmaxf(big, x);
+      for (int r = 0; r < 16; r += 2) {
+        const float x = acc[i][j][r], y = acc[i][j][r + 1];
+        most = max3_abs(most, x, y);
+        least = min(least, min((__float_as_uint(x) << 1) - 1u, (__float_as_uint(y) << 1) - 1u));
       }
-  // (per wave, its quarter of the tile: no barrier below)
-  if (__ballot(!finite) != 0 || (__ballot(big > 0.f) != 0 && __ballot(big >= 0x1p-64f) == 0)) {
+    }
+  bool again = __ballot(!(most < __builtin_inff())) != 0;
+  // (largest: of the operands' magnitudes)
+  auto doubtful = [&](float largest) {
+    const float bound = static_cast<float>(len) * fmaxf(largest * 0x1p-109f, 0x1p-99f);
+    return __ballot(least < (__float_as_uint(bound) << 1) - 1u) != 0;
+  };
+  if (len > 0) {
+    const uint4 look = *reinterpret_cast<const uint4*>(sLook);
+    if ((look.x | look.y | look.z | look.w) == 0u) {
+      again |= doubtful(kLarge);
+    } else {  // (the same for all waves)
+      for (int i = tid; i < BM + BN; i += kThreads) sTop[i] = 0u;
+      __syncthreads();
+      atomicMax(&sTop[oa.row[0]], __float_as_uint(topa));
+      atomicMax(&sTop[BM + ob.row[0]], __float_as_uint(topb));
+      __syncthreads();
+      // the rows and columns of the wave's quarter of the tile
+      const float ta = __uint_as_float(sTop[wm + lane % (BM / 2)]);
+      const float tb = __uint_as_float(sTop[BM + wn + lane % (BN / 2)]);
+      float m = fmaxf(ta, tb);
+#pragma unroll
+      for (int d = 32; d > 0; d /= 2) m = fmaxf(m, __shfl_xor(m, d));
+      again |= __ballot(tiny(ta) || tiny(tb)) != 0 || doubtful(m);
+    }
+  }
+  // (per wave: no barrier below)
+  if (again) {
     int ra[MT], rb[NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) ra[i] = min(wm + i * 32 + fr, g.M - 1 - m0);

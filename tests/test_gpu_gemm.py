@@ -237,3 +237,40 @@ def test_block_with_an_expanded_projection(cuda):
         out.append([y, *torch.autograd.grad(y.sum(), m.parameters())])
     for p, q in zip(*out):
         assert (p - q).abs().max() <= 1e-5 * q.abs().max()
+
+
+@pytest.mark.parametrize("akm,bkm", [(1, 1), (1, 0), (0, 1), (0, 0)])
+@pytest.mark.parametrize("k,splits", [(20, 1), (64, 1), (333, 3)])
+@pytest.mark.parametrize("kind", ["one row", "one column", "times large", "single terms", "subnormal row", "both small"])
+def test_tiny_values_beside_normal_ones(cuda, akm, bkm, k, splits, kind):
+    """Operands whose low parts are finer than bf16's smallest subnormal keep
+    float32's precision: (k + 4) roundings of 2^-23 S, S = sum |a b|, each of
+    at least half a float32 subnormal."""
+    m, n = 140, 70
+    gen = torch.Generator().manual_seed(k)
+    a, A, lda, _ = _operand(m, k, akm, 1, 0, gen)
+    b, B, ldb, _ = _operand(n, k, bkm, 1, 0, gen)
+    a, b = a[0], b[0]
+    if kind == "one row":
+        a[71] *= 2.0 ** -118
+    elif kind == "one column":
+        b[3] *= 2.0 ** -121
+    elif kind == "times large":
+        a *= 2.0 ** -118
+        b *= 2.0 ** 60
+    elif kind == "single terms":  # tiny values reach the result alone, in rows of normal ones
+        a[:, 5] *= 2.0 ** -120
+        b[9] = 0.0
+        b[9, 5] = 2.0 ** 90
+    elif kind == "subnormal row":
+        a[100] *= 2.0 ** -138
+        b *= 2.0 ** 20
+    else:
+        a *= 2.0 ** -60
+        b *= 2.0 ** -58
+    C = torch.empty(m, n, device="cuda")
+    d = _lib.GemmDesc(m, n, k, 1, lda, ldb, n, 0, 0, 0, 0, 0, akm, bkm, 0, splits)
+    _run(d, A, B, C)
+    ref = a.double() @ b.double().t().contiguous()
+    S = a.abs().double() @ b.abs().double().t().contiguous()
+    assert ((C.double() - ref).abs() <= (k + 4) * (2.0 ** -23 * S + 2.0 ** -149)).all()
