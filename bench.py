@@ -13,10 +13,10 @@ batch 32 of 224x224x1 images ~ N(0,1), patch 16 -> 196 tokens, embed_dim
 [1e-3, 1e-1]); loss = mean of the output features; one step = forward +
 loss + backward + AdamW update (the package's one-launch AdamW,
 mlx_vision_mamba_amd.optim; --torch-adamw for torch's fused AdamW).  The fp32
-projections run on the package's products (csrc/gemm.hip); dt_proj's two over
-the rows and the patch embedding use the TunableOp picks recorded for this step
-on MI355X (mlx_vision_mamba_amd/tuning/, read-only; --default-gemms for the
-library defaults).  Inputs are resident on the GPU before the
+projections run on the package's products (csrc/gemm.hip); the gradient
+of dt_proj's input and the patch embedding use the TunableOp picks recorded for
+this step on MI355X (mlx_vision_mamba_amd/tuning/, read-only; --default-gemms
+for the library defaults).  Inputs are resident on the GPU before the
 timed region; W untimed warm-up steps, then exactly K steps between two
 device synchronisations.  value = images / second.  The step is captured once
 in a HIP graph (after the warm-up) and the K timed steps are K replays of it,

@@ -708,19 +708,22 @@ mvm_gemm_desc gemm_desc(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ld
 
 constexpr int64_t kMaxLd = int64_t{1} << 21;
 
-// batch x rows from which dt_proj's products over the rows (delta_raw's
-// gradient, and delta_raw itself where the scan does not form it) are left to
-// the BLAS library: they stream 77 MB at 4 x 6272 rows of 768 channels, with
-// almost no arithmetic, and the library's picks take 22.3 and 25.6 us there,
-// the kernels here 27.3 and 31.4; at 8 x 1024 rows it is 20 and 21 us against
-// 13.7 and 12.1.
-constexpr int64_t kStreamRows = 16384;
+// Values of the streamed operand from which a `stream` product (delta_raw's
+// gradient times W_dt: every channel read once, a few columns out, hardly any
+// arithmetic) is left to the BLAS library.  Measured us, here / library with
+// its default picks, by MB streamed, at 128 to 3072 channels and 392 to 98304
+// rows: 25 MB and less 4-15 / 17-19 everywhere; 50 MB: 128 channels 18.3 / 18.2,
+// 768 18.3 / 18.6, 1536 21.3 / 20.1; 63-79 MB: 320 19.4 / 19.2, 768 26.1 / 20.7;
+// 101 MB: 1536 32.3 / 28.1, 3072 62 / 40; 126-157 MB: 320 34.8 / 26.1, 768 38.6 /
+// 35.0, 1536 48 / 53, 3072 66 / 76; 302 MB: 768 81 / 70, 1536 82 / 91, 3072 138 /
+// 127.  (The forward product is slower here in 2 of those 65 cases: it stays.)
+constexpr int64_t kStreamValues = 12 << 20;
 
 // out[q] (+)= op(A[q]) @ op(B[q]) for float32 (batch, rows, cols) views; ta /
 // tb transpose an operand.  The kernels take contiguous columns, operand rows
 // that do not overlap, and 16-byte rows of an operand whose summed index is the
 // contiguous one (from 32 summed values up); other operands (a parameter that
-// is an expanded row, say), and `stream` products of many rows, are torch's.
+// is an expanded row, say), and `stream` products from kStreamValues, are torch's.
 void batched(const Tensor& A, const Tensor& B, Tensor& out, bool ta, bool tb, bool accumulate, bool stream) {
   TORCH_CHECK(A.dim() == 3 && B.dim() == 3 && out.dim() == 3, "batched products take 3-D tensors");
   const int64_t q = A.size(0), m = A.size(ta ? 2 : 1), k = A.size(ta ? 1 : 2), n = B.size(tb ? 1 : 2);
@@ -733,7 +736,7 @@ void batched(const Tensor& A, const Tensor& B, Tensor& out, bool ta, bool tb, bo
   auto rows16 = [](const Tensor& t) { return t.stride(1) % 4 == 0 && t.stride(0) % 4 == 0 && aligned16(t); };
   auto rows = [](const Tensor& t) { return t.stride(2) == 1 && t.stride(1) >= t.size(2) && t.stride(1) < kMaxLd; };
   const bool ok = rows(A) && rows(B) && out.stride(2) == 1 && (k < 32 || ((ta || rows16(A)) && (!tb || rows16(B)))) &&
-                  !(stream && q * m > kStreamRows);
+                  !(stream && q * m * k >= kStreamValues);
   if (ok) {
     auto d = gemm_desc(m, n, k, A.stride(1), B.stride(1), out.stride(1), !ta, tb);
     d.batch = q;
@@ -989,15 +992,14 @@ struct CoreFn : Function<CoreFn> {
     Tensor dbc = padded_rows(K, M, R + 2 * ns, xz);
     batched(xc, W_x, dbc, false, true, false, false);                                  // :174
     const Tensor bc = bnkd(dbc, bsz, n);
-    // dt_proj (:180) inside the scan, up to its largest rank; else, and when
-    // delta_raw of many rows is kept for the backward, as a product (writing
-    // it from the scan costs there what the product does: 4 x 6272 rows
-    // trained 1542 us a block step inside, 1534 with the product; forward
-    // only, 8 x 1024 rows, 1289 us an encoder pass inside, 1314 with it)
-    const bool dt_in = R <= MVM_SCAN_MAX_DT_RANK && W_dt.is_contiguous() && !(save && K * M > kStreamRows);
+    // dt_proj (:180) inside the scan, up to its largest rank, else as a product
+    // (which writes delta_raw for the scan to read: block steps of 4 x 6272
+    // rows of 768 channels 1529 us inside, 1526 with the product; of 6 x 16384
+    // rows 5985 and 6043; an encoder's forward of 8 x 1024 rows 1289 and 1314)
+    const bool dt_in = R <= MVM_SCAN_MAX_DT_RANK && W_dt.is_contiguous();
     // (forward only: delta_raw is never formed in memory; xc lends its layout)
     Tensor delta_raw = dt_in && !save ? xc : empty_like_opts({K, M, din}, xz);
-    if (!dt_in) batched(dbc.narrow(2, 0, R), W_dt, delta_raw, false, true, false, true);
+    if (!dt_in) batched(dbc.narrow(2, 0, R), W_dt, delta_raw, false, true, false, false);
     // (the products of a block round more than its scan does)
     if (chunk_len == 0) {
       const auto d = make_desc(bnkd(xc, bsz, n), bc.narrow(3, R, ns), at::kFloat, at::kFloat, tok, 0);

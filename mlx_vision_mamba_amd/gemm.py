@@ -34,6 +34,6 @@ def batched(A, B, out=None, ta=False, tb=False, accumulate=False, stream=False):
     """out[q] (+)= op(A[q]) @ op(B[q]) for float32 (batch, rows, cols) views;
     ta / tb transpose an operand.  The kernels take contiguous columns, and
     16-byte rows of an operand whose summed index is the contiguous one (from
-    32 summed values up); for other operands, and for a ``stream`` product of
-    many rows, torch computes it."""
+    32 summed values up); for other operands, and for a ``stream`` product that
+    reads 12 Mi values of A or more, torch computes it."""
     return _lib.native().batched(A, B, out, ta, tb, accumulate, stream)

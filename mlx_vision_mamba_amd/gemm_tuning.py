@@ -1,11 +1,12 @@
 """GEMM selections for the VisionMamba projections on MI355X.
 
-dt_proj's products over many rows, and projections of shapes that the HIP
-products do not take (gemm.py), are plain fp32 GEMMs on the ROCm BLAS libraries.  PyTorch's
-TunableOp can pick, per GEMM shape, the fastest of the rocBLAS and
+The gradient of dt_proj's input over many rows, and projections of shapes that
+the HIP products do not take (gemm.py), are plain fp32 GEMMs on the ROCm BLAS
+libraries.  PyTorch's TunableOp can pick, per GEMM shape, the fastest of the rocBLAS and
 hipBLASLt solutions; ``tuning/gemm_mi355x_visionmamba2d.csv`` holds the
 picks measured on MI355X for the VisionMamba-2D training step (batch 32,
-224x224x1, patch 16, E = 384, K = 4).  ``load()`` turns TunableOp on in
+224x224x1, patch 16, E = 384, K = 4), those of products that run on the HIP
+kernels now among them.  ``load()`` turns TunableOp on in
 read-only mode with that file: listed shapes use the recorded solution,
 other shapes keep the library default, and nothing is tuned at run time.
 The file's validator lines (PyTorch, HIP, hipBLASLt, rocBLAS versions,

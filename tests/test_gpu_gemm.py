@@ -274,3 +274,28 @@ def test_tiny_values_beside_normal_ones(cuda, akm, bkm, k, splits, kind):
     ref = a.double() @ b.double().t().contiguous()
     S = a.abs().double() @ b.abs().double().t().contiguous()
     assert ((C.double() - ref).abs() <= (k + 4) * (2.0 ** -23 * S + 2.0 ** -149)).all()
+
+
+@pytest.mark.parametrize("m", [4095, 4096])
+def test_streamed_product_on_both_sides_of_its_rule(cuda, m):
+    """delta_raw's gradient times W_dt, 4 x m rows of 768 channels: the
+    kernels below 12 Mi streamed values, torch from there on."""
+    gen = torch.Generator().manual_seed(m)
+    a, b = [torch.randn(*s, generator=gen).cuda() for s in ((4, m, 768), (4, 768, 24))]
+    out = torch.empty(4, m, 56, device="cuda")
+    gemm.batched(a, b, out=out[..., :24], stream=True)
+    ref, S = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    # (any order of 768 float32 additions; both are far below it)
+    assert ((out[..., :24].double() - ref).abs() <= 770 * 2.0 ** -24 * S).all()
+
+
+def test_training_and_inference_form_delta_alike(cuda):
+    """A block of more than 16384 batch x rows: the same output bit for bit
+    with and without gradients."""
+    import mlx_vision_mamba_amd as mvm
+    torch.manual_seed(0)
+    m = mvm.MambaBlock(48, d_state=4, scan_mode="hip").to(cuda)
+    x = torch.randn(9, 1900, 48, generator=torch.Generator().manual_seed(1)).to(cuda)
+    y = m(x)
+    with torch.no_grad():
+        assert torch.equal(m(x), y)
