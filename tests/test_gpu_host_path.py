@@ -317,3 +317,20 @@ def test_error_types_of_a_backward(cuda, which, change, error, match):
     assert type(e.value) is error
     if error is _lib.ScanError:
         assert e.value.code == _lib.MVM_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("shape", [(0, 9, 2, 8), (2, 0, 2, 8), (1, 1, 1, 8), (3, 1, 2, 8)])
+def test_conv_backward_of_an_expanded_gradient(cuda, shape):
+    """The gradient of a sum is expanded: strides of zero, which an empty
+    tensor keeps through contiguous()."""
+    gen = torch.Generator().manual_seed(1)
+    x = torch.randn(*shape, generator=gen).to(cuda).requires_grad_()
+    w = torch.randn(shape[2], 8, 4, generator=gen).to(cuda).requires_grad_()
+    b = torch.randn(shape[2], 8, generator=gen).to(cuda).requires_grad_()
+    got = torch.autograd.grad(causal_conv_silu(x, w, b).sum(), (x, w, b))
+    xd, wd, bd = [t.detach().double().cpu().requires_grad_() for t in (x, w, b)]
+    pad = torch.nn.functional.pad(xd, (0, 0, 0, 0, 3, 0))
+    z = sum(pad[:, j:j + shape[1]] * wd[..., j] for j in range(4)) + bd
+    ref = torch.autograd.grad(torch.nn.functional.silu(z).sum(), (xd, wd, bd))
+    for a, r in zip(got, ref):
+        assert a.shape == r.shape and torch.allclose(a.double().cpu(), r, rtol=1e-5, atol=1e-5)
