@@ -791,7 +791,9 @@ struct InProjFn : Function<InProjFn> {
     const Tensor& W = sv[1];
     const int64_t O = W.size(0), E = W.size(1);
     Tensor dh, dW;
-    if (at::GradMode::is_enabled()) {  // create_graph: products that have a derivative themselves
+    // create_graph, or gradients batched by vmap (is_grads_batched): torch's
+    // products, which have a derivative and a batching rule
+    if (at::GradMode::is_enabled() || !g[0].has_storage()) {
       if (ctx->needs_input_grad(0)) dh = at::matmul(g[0], W);
       if (ctx->needs_input_grad(1)) dW = at::matmul(g[0].reshape({-1, O}).t(), sv[0].reshape({-1, E}));
       return {dh, dW};
@@ -846,7 +848,7 @@ struct OutProjFn : Function<OutProjFn> {
     const int64_t K = W.size(0), E = W.size(1), D = W.size(2);
     Tensor dy, dW;
     const Tensor dres = ctx->saved_data["res"].toBool() ? g[0] : Tensor();
-    if (at::GradMode::is_enabled()) {  // as in InProjFn
+    if (at::GradMode::is_enabled() || !g[0].has_storage()) {  // as in InProjFn
       const Tensor Wc = W.permute({1, 0, 2}).reshape({E, K * D});
       if (ctx->needs_input_grad(0)) dy = at::matmul(g[0], Wc).view(ctx->saved_data["shape"].toIntVector());
       if (ctx->needs_input_grad(1))

@@ -334,3 +334,19 @@ def test_conv_backward_of_an_expanded_gradient(cuda, shape):
     ref = torch.autograd.grad(torch.nn.functional.silu(z).sum(), (xd, wd, bd))
     for a, r in zip(got, ref):
         assert a.shape == r.shape and torch.allclose(a.double().cpu(), r, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("cls", [mvm.MambaBlock, mvm.ResidualMambaBlock])
+def test_batched_gradients_of_out_proj(cuda, cls):
+    """A Jacobian's rows in one vmapped backward, as far as out_proj's weight."""
+    torch.manual_seed(0)
+    m = cls(32, d_state=4, scan_mode="hip").to(cuda)
+    w = getattr(m, "mamba", m).out_proj.weight
+    gen = torch.Generator().manual_seed(1)
+    y = m(torch.randn(2, 20, 32, generator=gen).to(cuda))
+    v = torch.randn(3, 2, 20, 32, generator=gen).to(cuda)
+    (got,) = torch.autograd.grad(y, w, v, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        (ref,) = torch.autograd.grad(y, w, v[i], retain_graph=True)
+        # (40 terms in any order)
+        assert (got[i] - ref).abs().max() <= 1e-5 * ref.abs().max()
