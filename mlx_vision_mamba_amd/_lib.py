@@ -225,10 +225,15 @@ class _TracedCall(torch.autograd.Function):
         return tuple(res)
 
 
-def call(fn, *args):
-    """``fn(*args)``, through a node that the tracer keeps while one is at
-    work.  ``fn`` is a module-level function over the C++ host path."""
-    return _TracedCall.apply(fn, *args) if torch.jit.is_tracing() else fn(*args)
+# whether torch.jit.trace is recording: asked on every call of the host path, so
+# without the scripting check of torch.jit.is_tracing
+is_tracing = torch._C._is_tracing
+
+
+def traced(fn, *args):
+    """``fn(*args)`` as a node that the tracer keeps; ``fn`` is a module-level
+    function over the C++ host path."""
+    return _TracedCall.apply(fn, *args)
 
 
 def last_error() -> str:

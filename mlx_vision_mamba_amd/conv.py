@@ -32,4 +32,6 @@ def causal_conv_silu(x, weight, bias, seq_to_tok=None):
         if seq_to_tok.dtype != torch.int32 or seq_to_tok.shape != (x.shape[2], x.shape[1]):
             raise ValueError("seq_to_tok must be int32 of shape (K, N)")
         seq_to_tok = seq_to_tok.to(x.device).contiguous()
-    return _lib.call(_conv_silu, x, weight, bias, seq_to_tok)
+    if _lib.is_tracing():
+        return _lib.traced(_conv_silu, x, weight, bias, seq_to_tok)
+    return _conv_silu(x, weight, bias, seq_to_tok)

@@ -617,8 +617,9 @@ struct ConvFn : Function<ConvFn> {
     {
       at::NoGradGuard no_grad;
       Tensor dx = empty_like_opts(sv[0].sizes(), sv[0]);
-      // (dx's strides: one with no elements counts as contiguous whatever its own)
-      const Tensor dy = g[0].to(at::kFloat).contiguous().as_strided(dx.sizes(), dx.strides());
+      Tensor dy = g[0].to(at::kFloat).contiguous();
+      // (one with no elements counts as contiguous whatever its strides)
+      if (dy.strides() != dx.strides()) dy = dy.as_strided(dx.sizes(), dx.strides());
       auto [dw, db] = conv_bwd(sv[0], sv[1], sv[2], dy, dx, sv[3]);
       out = {dx, dw, db, Tensor()};
     }

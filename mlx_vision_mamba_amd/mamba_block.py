@@ -219,8 +219,8 @@ def _direction_stacks(owner, blocks):
     one per name of STACKED_PARAMS, kept on ``owner``.  Rebuilt (values
     copied from the current parameters, which then become slices of the new
     buffers) when any parameter is not its slice.  The per-call check
-    compares each parameter's data pointer, shape and dtype with those its
-    slice was given (the buffers are held here, so their memory is never
+    compares each parameter's data pointer, shape, strides, dtype and device
+    with its slice's (the buffers are held here, so their memory is never
     reused while the pointers are compared)."""
     return _stacks_of(owner, _params_of(blocks))
 
@@ -315,10 +315,16 @@ def _directional_forward(blocks, h, tok, scan_mode, owner=None, stacked=None, re
         stacks = _stacks_of(owner, params)
     flat = [p for ps in params for p in ps[:K]]
     # the reference's "metal" mode is inference only (mamba_metal.py:230)
-    return _lib.call(_directional, h, residual, tok, K, mode_chunk_len(scan_mode), scan_mode == "metal",
-                     len(flat), *flat, *stacks)
+    args = mode_chunk_len(scan_mode), scan_mode == "metal"
+    if _lib.is_tracing():
+        return _lib.traced(_directional_flat, h, residual, tok, K, *args, len(flat), *flat, *stacks)
+    return _directional(h, residual, tok, K, *args, flat, stacks)
 
 
-def _directional(h, residual, tok, K, chunk_len, detach, nparam, *tensors):
-    return _lib.native().directional(h, list(tensors[:nparam]), list(tensors[nparam:]), K, tok,
-                                     _resolve_chunk(h.shape[1], chunk_len), detach, residual)
+def _directional(h, residual, tok, K, chunk_len, detach, params, stacks):
+    return _lib.native().directional(h, params, stacks, K, tok, _resolve_chunk(h.shape[1], chunk_len), detach,
+                                     residual)
+
+
+def _directional_flat(h, residual, tok, K, chunk_len, detach, nparam, *tensors):
+    return _directional(h, residual, tok, K, chunk_len, detach, list(tensors[:nparam]), list(tensors[nparam:]))

@@ -31,7 +31,9 @@ class _LayerNormFn:
 
     @staticmethod
     def apply(x, weight, bias, eps, residual):
-        return _lib.call(_norm, x, weight, bias, eps, residual)
+        if _lib.is_tracing():
+            return _lib.traced(_norm, x, weight, bias, eps, residual)
+        return _norm(x, weight, bias, eps, residual)
 
 
 def layer_norm(x, norm, residual=False):

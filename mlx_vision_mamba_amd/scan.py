@@ -106,17 +106,6 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
-def _check_device(*ts):
-    dev = ts[0].device
-    if dev.type != "cuda":
-        raise RuntimeError(
-            "mlx_vision_mamba_amd scans run only on the GPU (HIP); got tensors on "
-            f"{dev}. There is no CPU fallback.")
-    for t in ts:
-        if t is not None and t.device != dev:
-            raise RuntimeError(f"all scan tensors must be on {dev}; got one on {t.device}")
-
-
 def _make_desc(u, Bm, in_dt, out_dt, tok, chunk_len):
     bsz, L, K, D = u.shape
     N = Bm.shape[-1]
@@ -232,7 +221,11 @@ def selective_scan_directions(u, delta, A, B, C, D, seq_to_tok=None, chunk_len=0
         y, _ = scan_forward(u.detach(), delta.detach(), A.detach(), B.detach(), C.detach(),
                             D.detach(), seq_to_tok, _resolve_chunk(u.shape[1], chunk_len), out_dtype)
         return y
-    return _lib.call(_scan, u, delta, A, B, C, D, seq_to_tok, chunk_len, out_dtype, False)
+    return _apply_scan(u, delta, A, B, C, D, seq_to_tok, chunk_len, out_dtype, False)
+
+
+def _apply_scan(*args):
+    return _lib.traced(_scan, *args) if _lib.is_tracing() else _scan(*args)
 
 
 def _scan(u, delta, A, B, C, D, tok, chunk_len, out_dtype, flat):
@@ -242,7 +235,7 @@ def _scan(u, delta, A, B, C, D, tok, chunk_len, out_dtype, flat):
 def _scan3(x, delta, A, B, C, D, chunk_len, out_dtype=None):
     if x.dim() != 3:
         raise ValueError(f"x must be (B, L, D); got {tuple(x.shape)}")
-    return _lib.call(_scan, x, delta, A, B, C, D, None, chunk_len, out_dtype, True)
+    return _apply_scan(x, delta, A, B, C, D, None, chunk_len, out_dtype, True)
 
 
 def selective_scan(x, delta, A, B, C, D, chunk_len=0, out_dtype=None):
