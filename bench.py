@@ -687,7 +687,9 @@ def main():
         "algorithmic_bytes_per_launch": int(bwd_b), "avg_launch_us": round(bwd_t * 1e6, 2),
         "launches": len(bwd),
         "fwd_call": {"achieved": round(fwd_b / fwd_t / 1e9, 1), "avg_launch_us": round(fwd_t * 1e6, 2),
-                     "algorithmic_bytes_per_launch": int(fwd_b)},
+                     "algorithmic_bytes_per_launch": int(fwd_b),
+                     # dt_proj's product inside: it writes delta_raw where the bytes count a read of it
+                     "includes": "dt_proj (mvm_scan_fused_dt_fwd)"},
         # the backward is VALU-issue bound: share of the kernel's time the
         # SIMDs' VALU is issuing (VALUBusy counter, committed profile)
         "valu_busy_per_simd": measured_traffic("bwd_valu_busy_per_simd", float),

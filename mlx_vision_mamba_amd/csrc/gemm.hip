@@ -3,8 +3,10 @@
 // mamba_block.py:125, :153, :165, :191).
 //
 // Why not the float32 matrix instructions: they reach 155 TFLOP/s on this
-// chip, the bf16 ones 1,700-1,800 from registers.  Every float32 x is the
-// exact sum of three bf16 values
+// chip, the bf16 ones 1,700-1,800 from registers.  The method is a published
+// one (Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations", 2019): every
+// float32 x is the exact sum of three bf16 values
 //   hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid    (round to nearest)
 // (24 = 8 + 8 + 8 significand bits), and
 //   a b = hi hi + (hi mid + mid hi) + (mid mid + hi lo + lo hi) + r,
@@ -57,8 +59,10 @@
 // neighbouring lanes share a bank.
 // Bound: with the MFMAs alone the loop runs at 230-240 TFLOP/s; the
 // split's VALU work (11 instructions per pair of values), the LDS traffic and
-// the global loads take the rest: 143-170 TFLOP/s on in_proj and out_proj of
-// 6272-16384 rows, where the BLAS library's float32 kernels reach 95-137.
+// the global loads take the rest: 135-170 TFLOP/s on in_proj and out_proj of
+// 6272-16384 rows, where the BLAS library's float32 kernels reach 95-137 (MFMA
+// pipes busy 39-47 % of the cycles, the VALU 29-37 %, LDS 20-24 %; the waves
+// wait to issue for half of theirs).
 // Scheduling barriers and raised wave priority around the MFMAs were both
 // slower (they keep the split's instructions from filling in between).
 //

@@ -42,7 +42,8 @@
 // further ahead than the rest.  It replaces a product that wrote delta_raw to
 // HBM and the scan's reading of it: one-image block forward 58.1 -> 51.7 us,
 // 4D encoder forward 1314 -> 1289, batch-2 block step 331 -> 289.  When
-// training, delta_raw is written from here for the backward.
+// training, delta_raw is written from here for the backward (at 4 x 6272 rows
+// of 768 channels 143 us, the scan and its product 115.5 + 25).
 #include "scan_common.h"
 #include "scan_kernels.h"
 
